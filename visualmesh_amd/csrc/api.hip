@@ -150,7 +150,7 @@ struct vmhip_batch {
      * wait for its copies */
     void* h_stage = nullptr;
     size_t h_stage_cap = 0;
-    void* h_pack = nullptr; /* pinned home of the segment table of a packed fetch */
+    void* h_pack = nullptr; /* pinned home of the chunk table of a packed fetch */
     size_t h_pack_cap = 0;
     bool stage_pending = false; /* copies of the last stage may still be reading h_stage (and the caller's images) */
     bool have_run = false;
@@ -887,15 +887,16 @@ int batch_fetch_packed_enqueue(vmhip_batch* b, void* block, size_t bytes, vmhip_
     std::vector<size_t> offsets;
     const size_t total = packed_layout(b, &offsets);
     if (bytes < total) return fail(VMHIP_ERR_CAPACITY, "fetch_packed: the block is smaller than vmhip_batch_fetch_packed_size says");
-    const size_t table_bytes = sizeof(VmPackSegment) * size_t(n) * 4;
+    const size_t most_chunks = total / VM_PACK_CHUNK + size_t(n) * 4; /* an array's last chunk is its only partial one */
+    const size_t table_bytes = sizeof(VmPackChunk) * most_chunks;
     if (table_bytes > b->h_pack_cap) {
         if (b->h_pack) HIP_TRY(hipHostFree(b->h_pack));
         b->h_pack = nullptr, b->h_pack_cap = 0;
-        HIP_TRY(hipHostMalloc(&b->h_pack, table_bytes, hipHostMallocDefault));
-        b->h_pack_cap = table_bytes;
+        HIP_TRY(hipHostMalloc(&b->h_pack, table_bytes + table_bytes / 4, hipHostMallocDefault));
+        b->h_pack_cap = table_bytes + table_bytes / 4;
     }
-    VmPackSegment* seg = static_cast<VmPackSegment*>(b->h_pack);
-    int n_seg = 0, n_chunks = 0;
+    VmPackChunk* const chunks = static_cast<VmPackChunk*>(b->h_pack);
+    int n_chunks = 0;
     uint8_t* host = static_cast<uint8_t*>(block);
     for (int f = 0; f < n; ++f) {
         const VmFrame& d = b->frames[f].dev;
@@ -907,8 +908,8 @@ int batch_fetch_packed_enqueue(vmhip_batch* b, void* block, size_t bytes, vmhip_
         const size_t base = size_t(d.row_base), stride = size_t(b->dev.nb_stride);
         const size_t* at = &offsets[size_t(f) * 4];
         auto add = [&](const void* src, size_t dst_offset, size_t nbytes, size_t row_bytes, size_t src_stride) {
-            seg[n_seg++] = VmPackSegment{static_cast<const uint8_t*>(src), dst_offset, nbytes, row_bytes, src_stride, n_chunks};
-            n_chunks += int((nbytes + VM_PACK_CHUNK - 1) / VM_PACK_CHUNK);
+            for (size_t begin = 0; begin < nbytes; begin += VM_PACK_CHUNK)
+                chunks[n_chunks++] = VmPackChunk{static_cast<const uint8_t*>(src), dst_offset, begin, std::min(begin + VM_PACK_CHUNK, nbytes), row_bytes, src_stride};
         };
         add(b->dev.row_px + base, at[0], 8 * V, 8, 8);
         add(b->dev.row_gidx + base, at[1], 4 * V, 4, 4);
@@ -924,11 +925,11 @@ int batch_fetch_packed_enqueue(vmhip_batch* b, void* block, size_t bytes, vmhip_
     if (total == 0) return VMHIP_OK;
     /* the kernel reads the table where it lies, in page-locked host memory: an upload would wait in the copy engine's
      * queue behind the images another engine is staging. The table is not touched again before vmhip_batch_fetch_wait. */
-    void* seg_dev = nullptr;
-    HIP_TRY(hipHostGetDevicePointer(&seg_dev, seg, 0));
+    void* chunks_dev = nullptr;
+    HIP_TRY(hipHostGetDevicePointer(&chunks_dev, chunks, 0));
     uint8_t* const direct = total <= PACK_DIRECT_MOST ? device_view(block) : nullptr;
     if (!direct) HIP_TRY(b->d_fetch_packed.reserve(total));
-    vm_launch_fetch_pack(static_cast<const VmPackSegment*>(seg_dev), n_seg, n_chunks, direct ? static_cast<void*>(direct) : b->d_fetch_packed.p, s);
+    vm_launch_fetch_pack(static_cast<const VmPackChunk*>(chunks_dev), n_chunks, direct ? static_cast<void*>(direct) : b->d_fetch_packed.p, s);
     HIP_TRY(hipGetLastError());
     if (!direct) HIP_TRY(hipMemcpyAsync(block, b->d_fetch_packed.p, total, hipMemcpyDeviceToHost, s));
     return VMHIP_OK;

@@ -210,15 +210,14 @@ void vm_detect_carve(void* workspace, size_t rows, int n_frames, VmDetectDev* D)
 void vm_launch_detect(const VmBatchDev& B, const VmDetectDev& D, int clusters, hipStream_t stream);
 /* packed: 5 * total_d + 7 * total_c words (detect.hip says in which order) */
 void vm_launch_detect_pack(const VmBatchDev& B, const VmDetectDev& D, uint32_t* packed, int total_d, int total_c, hipStream_t stream);
-/* one array of one frame on its way into the block of vmhip_batch_fetch_packed_async (detect.hip: vm_fetch_pack_kernel) */
+/* a piece of one array of one frame on its way into the block of vmhip_batch_fetch_packed_async (detect.hip: vm_fetch_pack_kernel) */
 #define VM_PACK_CHUNK 16384
-struct VmPackSegment {
-    const uint8_t* src;
-    size_t dst_offset, bytes;        /* multiples of 256 and of 4 */
+struct VmPackChunk {
+    const uint8_t* src;              /* the array; the chunk is its bytes begin .. end, at most VM_PACK_CHUNK of them */
+    size_t dst_offset, begin, end;   /* where the array goes: a multiple of 256; multiples of VM_PACK_CHUNK and of 4 */
     size_t row_bytes, src_stride;    /* equal for a contiguous array */
-    int32_t chunk_first;             /* number of the segment's first chunk of VM_PACK_CHUNK bytes */
 };
-void vm_launch_fetch_pack(const VmPackSegment* segments, int n_segments, int n_chunks, void* dst, hipStream_t stream);
+void vm_launch_fetch_pack(const VmPackChunk* chunks, int n_chunks, void* dst, hipStream_t stream);
 
 /* "<family>_<c_in>x<c_out>s<slots>" as a string that stays valid (the profile of a run names its kernels) */
 const char* vm_kernel_name(const char* family, int c_in, int c_out, int slots);
