@@ -243,7 +243,10 @@ int vmhip_batch_fetch_packed_async(vmhip_batch* batch, void* block, size_t bytes
 
 /* The fetch for callers that copy the results into memory of their own: results[i] is filled in as by
  * vmhip_batch_fetch_packed_async, with pointers into a block that belongs to the batch. Waits; the arrays stay as they are until
- * the next call of this function on the batch or the batch's end. No counterpart in the reference. */
+ * the next call of this function on the batch or the batch's end. Up to VMHIP_HELD_MOST bytes of results the block is page-locked and
+ * kept for the next call; for more (vmhip_batch_fetch_packed_size says how many there are) it is ordinary memory made for the call
+ * and given back by the next one: a caller that has arrays of its own uses vmhip_batch_fetch there. No counterpart in the reference. */
+#define VMHIP_HELD_MOST ((size_t) 64 << 20)
 int vmhip_batch_fetch_held(vmhip_batch* batch, vmhip_result* results);
 /* vmhip_project with its results in a block that belongs to the engine, until the engine's next vmhip_project_held */
 int vmhip_project_held(vmhip_engine* engine, const vmhip_frame* frame, vmhip_result* result);

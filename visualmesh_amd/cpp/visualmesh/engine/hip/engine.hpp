@@ -41,6 +41,7 @@
 #include <exception>
 #include <thread>
 #include <cstring>
+#include <limits>
 #include <map>
 #include <memory>
 #include <stdexcept>
@@ -166,28 +167,52 @@ namespace engine {
                                                                           const mat4<Scalar>& Hoc,
                                                                           const Lens<Scalar>& lens) const {
                 constexpr int N = Model<Scalar>::N_NEIGHBOURS;
-                const vmhip_result r = project_held(mesh, Hoc, lens);
+                FrameData fd;
+                find_ranges(mesh, Hoc, lens, fd);
+                describe(mesh, Hoc, lens, nullptr, 0, fd);
                 ProjectedMesh<Scalar, N> out;
+                vmhip_result r{};
+                if (projection_bytes<N>(fd) > VMHIP_HELD_MOST) {
+                    /* more than the engine keeps a block for: straight into arrays of the lookup's size */
+                    out.pixel_coordinates.resize(fd.candidates);
+                    out.global_indices.resize(fd.candidates);
+                    out.neighbourhood.resize(size_t(fd.candidates) + 1);
+                    r.capacity = fd.candidates;
+                    point_into(out, r);
+                    throw_on_error(vmhip_project(handle(N), &fd.frame, &r));
+                    out.pixel_coordinates.resize(r.n_visible);
+                    out.global_indices.resize(r.n_visible);
+                    out.neighbourhood.resize(size_t(r.n_visible) + 1);
+                }
+                else if (fd.candidates > 0) {
+                    throw_on_error(vmhip_project_held(handle(N), &fd.frame, &r));
+                    if (r.n_visible > 0) take<N>(r, out);
+                }
                 if (r.n_visible == 0) {
                     /* nothing visible: no pixels, no indices, and the neighbourhood table is its null row alone, pointing
                      * at itself (reference engine/cpu/engine.hpp:127-143 with n_points = 0) */
                     std::array<int, N> null_row;
                     null_row.fill(0);
                     out.neighbourhood.assign(1, null_row);
-                    return out;
                 }
-                take<N>(r, out);
                 return out;
             }
             /// The same with the results left in a block of the engine's (see vmhip_project_held), which its next projection
-            /// overwrites: n_visible rows, and null pointers if that is zero.
+            /// overwrites: n_visible rows, and null pointers if that is zero. Where the lookup leaves room for more than `most`
+            /// bytes of results nothing is projected: n_visible is -1, capacity the number of nodes that the lookup names.
             template <template <typename> class Model>
-            vmhip_result project_held(const Mesh<Scalar, Model>& mesh, const mat4<Scalar>& Hoc, const Lens<Scalar>& lens) const {
+            vmhip_result project_held(const Mesh<Scalar, Model>& mesh, const mat4<Scalar>& Hoc, const Lens<Scalar>& lens,
+                                      size_t most = std::numeric_limits<size_t>::max()) const {
+                constexpr int N = Model<Scalar>::N_NEIGHBOURS;
                 FrameData fd;
                 find_ranges(mesh, Hoc, lens, fd);
-                describe(mesh, Hoc, lens, nullptr, 0, fd);
                 vmhip_result r{};
-                if (fd.candidates > 0) throw_on_error(vmhip_project_held(handle(Model<Scalar>::N_NEIGHBOURS), &fd.frame, &r));
+                if (projection_bytes<N>(fd) > most) {
+                    r.n_visible = -1, r.capacity = fd.candidates;
+                    return r;
+                }
+                describe(mesh, Hoc, lens, nullptr, 0, fd);
+                if (fd.candidates > 0) throw_on_error(vmhip_project_held(handle(N), &fd.frame, &r));
                 return r;
             }
             template <template <typename> class Model>
@@ -213,14 +238,16 @@ namespace engine {
                 return std::move(classify(one)[0]);
             }
             /// The same with the results left in a block of the engine's (see vmhip_batch_fetch_held), which its next fetch()
-            /// or classification overwrites: n_visible rows, and null pointers if that is zero.
+            /// or classification overwrites: n_visible rows, and null pointers if that is zero. More than `most` bytes of results
+            /// stay on the device, as after run(): n_visible is set, the pointers are null.
             template <template <typename> class Model>
             vmhip_result classify_held(const Mesh<Scalar, Model>& mesh, const mat4<Scalar>& Hoc, const Lens<Scalar>& lens,
-                                       const void* image, const uint32_t& format) const {
+                                       const void* image, const uint32_t& format, size_t most = std::numeric_limits<size_t>::max()) const {
                 stage(std::vector<Frame<Model>>(1, Frame<Model>{&mesh, Hoc, lens, image, format}));
                 run();
                 vmhip_result r{};
-                throw_on_error(vmhip_batch_fetch_held(batch_, &r));
+                if (packed_size() > most) r.n_visible = visible_counts()[0];
+                else throw_on_error(vmhip_batch_fetch_held(batch_, &r));
                 return r;
             }
             template <template <typename> class Model>
@@ -321,6 +348,24 @@ namespace engine {
                 if (n == 0) return out;
                 const int classes = vmhip_engine_n_classes(engine_);
                 std::vector<vmhip_result> results(n);
+                if (packed_size() > VMHIP_HELD_MOST) {
+                    /* more than the batch keeps a block for: every array straight to its vector */
+                    const std::vector<int32_t> visible = visible_counts();
+                    for (size_t i = 0; i < n; ++i) {
+                        const size_t V = size_t(visible[i]);
+                        results[i] = vmhip_result{};
+                        results[i].capacity = visible[i];
+                        if (V == 0) continue;
+                        out[i].pixel_coordinates.resize(V);
+                        out[i].global_indices.resize(V);
+                        out[i].neighbourhood.resize(V + 1);
+                        out[i].classifications.resize((V + 1) * classes);
+                        point_into(out[i], results[i]);
+                        results[i].classifications = out[i].classifications.data();
+                    }
+                    throw_on_error(vmhip_batch_fetch(batch_, results.data()));
+                    return out;
+                }
                 throw_on_error(vmhip_batch_fetch_held(batch_, results.data()));
                 for (size_t i = 0; i < n; ++i) {
                     const vmhip_result& r = results[i];
@@ -601,6 +646,18 @@ namespace engine {
                 out.pixel_coordinates.assign(px, px + V);
                 out.global_indices.assign(r.global_indices, r.global_indices + V);
                 out.neighbourhood.assign(nb, nb + V + 1);
+            }
+            /// The arrays of `out` as the places that a download writes to.
+            template <typename Out>
+            static void point_into(Out& out, vmhip_result& r) {
+                r.pixel_coordinates = reinterpret_cast<float*>(out.pixel_coordinates.data());
+                r.global_indices = out.global_indices.data();
+                r.neighbourhood = reinterpret_cast<int32_t*>(out.neighbourhood.data());
+            }
+            /// What a projection of the nodes that the lookup names returns at most.
+            template <int N>
+            static size_t projection_bytes(const FrameData& fd) {
+                return size_t(fd.candidates) * (sizeof(std::array<Scalar, 2>) + sizeof(int32_t) + sizeof(std::array<int32_t, N>));
             }
             /// The host side of the path: the mesh's lookup, flattened for the C ABI. Touches nothing but `fd`.
             template <template <typename> class Model>

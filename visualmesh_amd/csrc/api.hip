@@ -8,6 +8,8 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <memory>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -200,15 +202,11 @@ struct vmhip_batch {
     DevBuf d_frames, d_ranges, d_images, d_cand_px, d_cand_g, d_cand_keep, d_tile_count, d_force_valid, d_force_keep, d_frame_V,
       d_amb_list, d_row_px, d_row_gidx, d_row_nb, d_row_nbl, d_tile_halo, d_tile_desc, d_row_nbl_h, d_tile_note_h, d_active_h, d_act[2], d_lookup, d_epoch, d_detect, d_detect_packed, d_lookup_ws, d_export, d_fetch_packed;
     std::vector<std::vector<int32_t>> device_ranges; /* per frame: the ranges a lookup on the device produced */
-    /* the results of vmhip_batch_fetch_held: page-locked up to HELD_PINNED_MOST bytes, else (or if none is to be had) plain memory */
+    /* the results of vmhip_batch_fetch_held: page-locked up to VMHIP_HELD_MOST bytes and kept, else (or if none is to be had) plain memory
+     * until the next call */
     void* h_held = nullptr;
     size_t h_held_cap = 0;
-    bool h_held_pinned = false;
-    void drop_held() {
-        if (h_held && h_held_pinned) (void) hipHostFree(h_held);
-        else std::free(h_held);
-        h_held = nullptr, h_held_cap = 0;
-    }
+    std::unique_ptr<uint8_t[]> h_held_plain;
     void* h_detect = nullptr; /* pinned landing area of vmhip_batch_detect */
     size_t h_detect_cap = 0;
     float* final_act = nullptr;
@@ -236,7 +234,9 @@ struct vmhip_batch {
         h_pack = nullptr, h_pack_cap = 0;
         if (h_detect) (void) hipHostFree(h_detect);
         h_detect = nullptr, h_detect_cap = 0;
-        drop_held();
+        if (h_held) (void) hipHostFree(h_held);
+        h_held = nullptr, h_held_cap = 0;
+        h_held_plain.reset();
         for (hipEvent_t e : events) (void) hipEventDestroy(e);
         events.clear();
     }
@@ -875,8 +875,9 @@ uint8_t* device_view(void* block) {
     return at.type == hipMemoryTypeHost && at.device == device && at.devicePointer == block ? static_cast<uint8_t*>(block) : nullptr;
 }
 
-/* vmhip_batch_fetch_packed_async: one kernel gathers every frame's arrays into one device block, one copy brings it home */
-int batch_fetch_packed_enqueue(vmhip_batch* b, void* block, size_t bytes, vmhip_result* results) {
+/* vmhip_batch_fetch_packed_async: one kernel gathers every frame's arrays, up to `direct_most` bytes straight into the caller's block (if
+ * it can be stored to), else into one device block that one copy brings home */
+int batch_fetch_packed_enqueue(vmhip_batch* b, void* block, size_t bytes, vmhip_result* results, size_t direct_most) {
     if (!b->have_run) return fail(VMHIP_ERR_ARGUMENT, "fetch: no completed run");
     if (!results || !block) return fail(VMHIP_ERR_ARGUMENT, "fetch_packed: null block or results");
     if (b->fetching) return fail(VMHIP_ERR_ARGUMENT, "fetch: a fetch of this batch is still in flight (vmhip_batch_fetch_wait first)");
@@ -927,7 +928,7 @@ int batch_fetch_packed_enqueue(vmhip_batch* b, void* block, size_t bytes, vmhip_
      * queue behind the images another engine is staging. The table is not touched again before vmhip_batch_fetch_wait. */
     void* chunks_dev = nullptr;
     HIP_TRY(hipHostGetDevicePointer(&chunks_dev, chunks, 0));
-    uint8_t* const direct = total <= PACK_DIRECT_MOST ? device_view(block) : nullptr;
+    uint8_t* const direct = total <= direct_most ? device_view(block) : nullptr;
     if (!direct) HIP_TRY(b->d_fetch_packed.reserve(total));
     vm_launch_fetch_pack(static_cast<const VmPackChunk*>(chunks_dev), n_chunks, direct ? static_cast<void*>(direct) : b->d_fetch_packed.p, s);
     HIP_TRY(hipGetLastError());
@@ -945,31 +946,54 @@ int batch_fetch(vmhip_batch* b, vmhip_result* results) {
 }
 
 /* vmhip_batch_fetch_held. Copies of a frame's four arrays into memory that is not page-locked each cost a submission, a wait and
- * the runtime's own staging; this is one kernel (and above PACK_DIRECT_MOST one copy) into a block that the batch keeps, from which
- * the caller copies once, into arrays of the right size. One call from host image to host arrays, before and now (the caller's
- * second lookup, made to size the arrays, is gone with it): 1280x1024 RGBA 770 / 448 us, Bayer with 128 000 nodes of eight
- * neighbours 1802 / 812, 320x256 204 / 150; a projection of a whole mesh of 9 000 nodes 605 / 349. */
-constexpr size_t HELD_PINNED_MOST = size_t(64) << 20; /* page-locked memory is the whole system's: a batch keeps no more of it */
+ * the runtime's own staging; this is one kernel that stores into a block that the batch keeps (whatever the size: no second copy of the
+ * results on the device, 1.6 % slower than one at 51 MB), from which the caller copies once, into arrays of the right size. fetch() in
+ * us, array by array / so: one frame of 3.4 MB 723 / 188, four (13 MB) 1070 / 670, sixteen (53 MB) 8100 / 7200. One call from host image
+ * to host arrays, with a second lookup to size them and array by array / so, and with the stage's one launch (project.hip): 1280x1024
+ * RGBA 755 / 450, Bayer with 128 000 nodes of eight neighbours 1682 / 795, 320x256 202 / 142; a projection of 9 000 nodes 613 / 323.
+ * Past VMHIP_HELD_MOST, or without page-locked memory, the arrays are copied one by one into plain memory; Engine::fetch() and the calls
+ * of one frame do not come here then, their arrays are copied straight to their places: 210 MB take 38.2 ms so, 44.4 through a plain block. */
 int batch_fetch_held(vmhip_batch* b, vmhip_result* results) {
     if (!b->have_run) return fail(VMHIP_ERR_ARGUMENT, "fetch: no completed run");
-    const size_t need = std::max<size_t>(packed_layout(b, nullptr), 256);
-    const bool pinned = need <= HELD_PINNED_MOST;
-    if (need > b->h_held_cap || (pinned && !b->h_held_pinned)) {
-        b->drop_held();
-        const size_t want = pinned ? std::min(need + need / 8, HELD_PINNED_MOST) : need;
-        b->h_held_pinned = pinned && hipHostMalloc(&b->h_held, want, hipHostMallocDefault) == hipSuccess;
-        if (!b->h_held_pinned) {
-            (void) hipGetLastError();
-            b->h_held = std::malloc(want);
+    if (!results) return fail(VMHIP_ERR_ARGUMENT, "fetch: null results");
+    if (b->fetching) return fail(VMHIP_ERR_ARGUMENT, "fetch: a fetch of this batch is still in flight (vmhip_batch_fetch_wait first)");
+    b->h_held_plain.reset();
+    std::vector<size_t> offsets;
+    const size_t need = std::max<size_t>(packed_layout(b, &offsets), 256);
+    if (need <= VMHIP_HELD_MOST && need > b->h_held_cap) {
+        if (b->h_held) HIP_TRY(hipHostFree(b->h_held));
+        b->h_held = nullptr, b->h_held_cap = 0;
+        const size_t want = std::min(need + need / 8, VMHIP_HELD_MOST);
+        if (hipHostMalloc(&b->h_held, want, hipHostMallocDefault) == hipSuccess) {
+            b->h_held_cap = want;
         }
-        if (!b->h_held) return fail(VMHIP_ERR_HIP, "fetch: out of host memory");
-        b->h_held_cap = want;
+        else {
+            (void) hipGetLastError();
+            b->h_held = nullptr;
+        }
     }
-    const int rc = batch_fetch_packed_enqueue(b, b->h_held, b->h_held_cap, results);
-    const hipError_t e = hipStreamSynchronize(b->engine->stream);
-    if (rc != VMHIP_OK) return rc;
-    HIP_TRY(e);
-    return VMHIP_OK;
+    if (need <= b->h_held_cap) {
+        const int rc = batch_fetch_packed_enqueue(b, b->h_held, b->h_held_cap, results, VMHIP_HELD_MOST);
+        const hipError_t e = hipStreamSynchronize(b->engine->stream);
+        if (rc != VMHIP_OK) return rc;
+        HIP_TRY(e);
+        return VMHIP_OK;
+    }
+    b->h_held_plain.reset(new (std::nothrow) uint8_t[need]);
+    if (!b->h_held_plain) return fail(VMHIP_ERR_HIP, "fetch: out of host memory");
+    for (size_t f = 0; f < b->frames.size(); ++f) {
+        vmhip_result& R = results[f];
+        uint8_t* const p = b->h_held_plain.get();
+        const size_t* at = &offsets[f * 4];
+        std::memset(&R, 0, sizeof(R));
+        R.capacity = b->h_V[f];
+        if (b->h_V[f] == 0) continue;
+        R.pixel_coordinates = reinterpret_cast<float*>(p + at[0]);
+        R.global_indices = reinterpret_cast<int32_t*>(p + at[1]);
+        R.neighbourhood = reinterpret_cast<int32_t*>(p + at[2]);
+        if (b->classify) R.classifications = reinterpret_cast<float*>(p + at[3]);
+    }
+    return batch_fetch(b, results);
 }
 
 int ensure_scratch(vmhip_engine* E) {
@@ -1479,7 +1503,7 @@ size_t vmhip_batch_fetch_packed_size(const vmhip_batch* b) {
 }
 int vmhip_batch_fetch_packed_async(vmhip_batch* b, void* block, size_t bytes, vmhip_result* results) {
     if (!b) return fail(VMHIP_ERR_ARGUMENT, "batch_fetch_packed_async: null batch");
-    const int rc = batch_fetch_packed_enqueue(b, block, bytes, results);
+    const int rc = batch_fetch_packed_enqueue(b, block, bytes, results, PACK_DIRECT_MOST);
     if (rc != VMHIP_OK) {
         (void) hipStreamSynchronize(b->engine->stream);
         return rc;

@@ -117,7 +117,14 @@ class Engine:
         m = self._pick(mesh, Hoc)
         H = np.ascontiguousarray(Hoc, dtype=np.float32)
         r = native.Result()
-        V = native.host_check(self._lib.vmh_engine_project_held(self.ptr, m.ptr, _fp(H), C.byref(lens), C.byref(r)))
+        native.host_check(self._lib.vmh_engine_project_held(self.ptr, m.ptr, _fp(H), C.byref(lens), C.byref(r)))
+        V = r.n_visible
+        if V < 0:  # more than the engine holds, perhaps: arrays for the lookup's nodes
+            cap = r.capacity
+            px, nb, gidx = np.empty((cap, 2), np.float32), np.empty((cap + 1, m.n_neighbours), np.int32), np.empty(cap, np.int32)
+            V = native.host_check(self._lib.vmh_engine_project(self.ptr, m.ptr, _fp(H), C.byref(lens), cap, _fp(px), _ip(nb), _ip(gidx)))
+            if V:
+                return dict(px=px[:V].copy(), nb=nb[:V + 1].copy(), gidx=gidx[:V].copy())
         nn = m.n_neighbours
         if V == 0:  # the neighbourhood table is its null row alone, as the reference's projection returns it
             return dict(px=np.zeros((0, 2), np.float32), nb=np.zeros((1, nn), np.int32), gidx=np.zeros(0, np.int32))
@@ -130,9 +137,15 @@ class Engine:
         n_out, nn = self.network.n_out, m.n_neighbours
         img = np.ascontiguousarray(image)
         r = native.Result()
-        V = native.host_check(self._lib.vmh_engine_classify_held(self.ptr, m.ptr, _fp(H), C.byref(lens), img.ctypes.data, fcc, C.byref(r)))
+        native.host_check(self._lib.vmh_engine_classify_held(self.ptr, m.ptr, _fp(H), C.byref(lens), img.ctypes.data, fcc, C.byref(r)))
+        V = r.n_visible
         if V == 0:
             return dict(px=np.zeros((0, 2), np.float32), nb=np.zeros((0, nn), np.int32), gidx=np.zeros(0, np.int32), cls=np.zeros((0, n_out), np.float32))
+        if not r.pixel_coordinates:  # more than the engine holds: straight from the device
+            px, nb, gidx, cls = np.empty((V, 2), np.float32), np.empty((V + 1, nn), np.int32), np.empty(V, np.int32), np.empty((V + 1, n_out), np.float32)
+            r = native.Result(V, 0, _fp(px), _ip(gidx), _ip(nb), _fp(cls))
+            native.hip_check(native.hip().vmhip_batch_fetch(self.native_batch(), C.byref(r)))
+            return dict(px=px, nb=nb, gidx=gidx, cls=cls)
         return dict(px=self._taken(r.pixel_coordinates, (V, 2), np.float32), nb=self._taken(r.neighbourhood, (V + 1, nn), np.int32),
                     gidx=self._taken(r.global_indices, (V,), np.int32), cls=self._taken(r.classifications, (V + 1, n_out), np.float32))
 
