@@ -491,7 +491,7 @@ namespace engine {
             }
             /// Where stage() looks up the nodes that may be on screen: on the host (Mesh::lookup, shared by a few
             /// threads; the default) or on the device, by a kernel that walks the same cone tree with the same
-            /// comparisons. The single-frame calls always use the host (they size their results by the lookup).
+            /// comparisons. A projection always uses the host's lookup; the classification of one frame is a batch of one.
             /// Needs a Mesh that exposes its cone tree (VISUALMESH_MESH_HAS_CONE_TREE); otherwise the host's lookup stays
 #if defined(VISUALMESH_MESH_HAS_CONE_TREE)
             void set_device_lookup(bool on) { device_lookup_ = on; }

@@ -859,7 +859,8 @@ size_t packed_layout(const vmhip_batch* b, std::vector<size_t>* offsets) {
 /* A packed fetch of up to this many bytes is stored into the caller's block by the packing kernel itself: the copy behind it is one
  * more submission, to another engine, and that costs more than the kernel's stores lose.
  * Fetches of configuration 2 in us, copied / stored: 3.4 MB 88 / 79, 7.3 MB 158 / 150, 11 MB 228 / 220, 25 MB 473 / 474, 51 MB
- * 951 / 966. The line lies well below the crossing: the stores occupy compute units that another engine's pass could use. */
+ * 951 / 966. Between 8 MB and the crossing the stores would gain 0 to 3 %; there the compute units are left to another engine's pass, a
+ * choice that has not been measured. */
 constexpr size_t PACK_DIRECT_MOST = size_t(8) << 20;
 
 /* the address by which a kernel on the current device reaches a block of page-locked host memory with 16-byte stores, or null:

@@ -232,7 +232,8 @@ __global__ __launch_bounds__(FLOW_WAVES * 64) void vm_conv_flow_kernel(VmBatchDe
      * consecutive row groups (a wave's 16 rows), one part per block; the block stages the whole tile, the waves of other
      * parts skip the contraction and the stores. Measured on 280
      * tiles (a frame of 71 645 rows: 24 tiles are left after the first round of 256 CUs), the six layers of 3-16-32 x 5-16-3
-     * and everything around them: 258.7 us before, 245.5 us now; 16 such frames (17.5 rounds) 1818 -> 1808. Four parts: a part
+     * and everything around them: 258.7 us before, 245.5 us now; 16 such frames (17.5 rounds) the same,
+     * 1795 to 1834 before and 1799 to 1823 now from run to run. Four parts: a part
      * then has one row group per SIMD, the least that costs less time. */
     auto scalar = [](int v) { return __builtin_amdgcn_readfirstlane(v); }; /* a division leaves its result in a vector register */
     const int n_xcd = max(t_end - xcd * per_xcd, 0);
