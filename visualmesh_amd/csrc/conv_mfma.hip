@@ -205,7 +205,11 @@ __global__ __launch_bounds__(NW * 64) void vm_conv_mfma_kernel(VmBatchDev B, VmL
             const v4u d = __builtin_amdgcn_raw_buffer_load_b128(desc_rsrc, tile * 16, 0, 0); /* {first row, rows in use, -, frame's first row} */
             const int tile_row0 = (int) d.x - (int) d.w;
             t.base = d.w;
-            t.V = tile_row0 + (int) d.y - 1; /* the last row in use: equals V in the frame's last tile, never clamps elsewhere */
+            /* the last row in use: equals V in the frame's last tile, never clamps in those before. A tile behind that one has no rows
+             * (a frame with many more candidates than visible nodes has such tiles): its lanes redo the frame's first row, which is always in
+             * use, and store nothing. The row before such a tile may never have been written, and a neighbour number read there may be
+             * anything. */
+            t.V = (int) d.y > 0 ? tile_row0 + (int) d.y - 1 : 0;
             t.row0 = tile_row0 + wave * (RB * 16);
         }
         else {
