@@ -251,7 +251,8 @@ int vmhip_batch_fetch_packed_async(vmhip_batch* batch, void* block, size_t bytes
  * as large as that fetch will need) stays alive and unused by the caller until vmhip_batch_fetch_wait of a packed fetch, or until the
  * announcement is withdrawn with a NULL block, which waits for the copy. A block that is too small or not page-locked, and a
  * fetch into another block or of another kind, are no errors: everything is then fetched as without an announcement.
- * vmhip_batch_delivered: the block that the last completed run has written to, or NULL. No counterpart in the reference. */
+ * vmhip_batch_delivered: the block that the last completed run has written to and that no packed fetch has followed, or NULL; a further fetch
+ * of the same run brings everything, whatever has become of the block. No counterpart in the reference. */
 int vmhip_batch_announce_packed(vmhip_batch* batch, void* block, size_t bytes);
 void* vmhip_batch_delivered(const vmhip_batch* batch);
 

@@ -141,3 +141,40 @@ def test_announcements_that_are_not_used():
         assert not lib.vmhip_batch_delivered(batch)
         got = engine.fetch_packed()
     _same(got, engine.fetch_pinned())
+
+
+def test_a_delivery_serves_one_fetch():
+    """What a packed fetch has brought is the caller's: changed in place, or its block freed and another one at the address, a further fetch
+    of the same run brings the run's results."""
+    lib, rng = native.hip(), np.random.default_rng(8)
+    engine = _engine()
+    engine.stage(_frames(rng, 2))
+    for _ in range(4):
+        engine.run()
+        want = _copied(engine.fetch_pinned())
+        for _ in range(3):
+            got = engine.fetch_packed()
+            _same(got, want)
+            for g in got:
+                g["px"] += 0.5
+                g["gidx"][:], g["nb"][:], g["cls"][:] = 7, -1, 0.0
+        engine.run()  # not fetched
+    batch = engine.native_batch()
+    need = int(lib.vmhip_batch_fetch_packed_size(batch))
+    for freed in (False, True):
+        block = native.pinned_empty((need,), np.uint8)
+        native.hip_check(lib.vmhip_batch_announce_packed(batch, block.ctypes.data, need))
+        engine.run()
+        assert lib.vmhip_batch_delivered(batch) == block.ctypes.data
+        for _ in range(2):
+            raw = (native.Result * 2)()
+            native.hip_check(lib.vmhip_batch_fetch_packed_async(batch, block.ctypes.data, need, raw))
+            native.hip_check(lib.vmhip_batch_fetch_wait(batch))
+            assert not lib.vmhip_batch_delivered(batch)
+            for r, w in zip(raw, want):
+                for pointer, key in ((r.pixel_coordinates, "px"), (r.global_indices, "gidx"), (r.neighbourhood, "nb"), (r.classifications, "cls")):
+                    assert np.array_equal(np.ctypeslib.as_array(pointer, w[key].shape), w[key]), (freed, key)
+            if freed:
+                del block
+                block = native.pinned_empty((need,), np.uint8)  # at the same address, as a rule
+            block[:] = 0xee
