@@ -136,14 +136,19 @@ def test_a_frame_alone_and_among_others(width):
 
 @pytest.mark.gpu
 def test_networks_whose_activations_could_leave_the_range():
-    """Weights by which a sum could reach 1e30, an infinite one, and activations without this kernel: the fp32 instructions, as ever."""
+    """Weights by which a sum could reach 1e30, infinite ones and such that are no numbers, whichever channel they belong to, and activations
+    without this kernel: the fp32 instructions, as ever."""
     frames = _frames(1, 1.5)
-    for change in ("large", "infinite", "tanh", "none"):
+    for change in ("large", "infinite", "nan", "infinite, then nan", "nan bias", "tanh", "none"):
         network = _network([3, 64, 64, 64, 4], wl.TANH if change == "tanh" else wl.SELU)
         if change == "large":
             network = [[(w * (1e14 if i in (0, 1) else 1), b, a) for w, b, a in g] for i, g in enumerate(network)]
-        if change == "infinite":
+        if change.startswith("infinite"):
             network[1][0][0][5, 7] = np.inf
+        if change.endswith("nan"):  # channels with finite sums follow
+            network[1][0][0][9, 8] = np.nan
+        if change == "nan bias":
+            network[1][0][1][30] = np.nan
         _, names = _run(eng.Engine(network, wl.RING6), frames)
         assert names.count("conv_x3_64x64s7") == (2 if change == "none" else 0), (change, names)
 
