@@ -926,7 +926,7 @@ __global__ __launch_bounds__(VMHIP_TILE, CB == 1 ? (NN <= 6 ? 8 : 6) : CB == 2 ?
         B.tile_desc[tile] = make_int4(row_base + row0, n_rows, min(total, cap), row_base);
         if (B.far_tiles && (total > VM_X3_TILE_HALO || total >= cap)) {
             const int at = atomicAdd(B.n_far_tiles, 1);
-            if (at < B.n_row_tiles) B.far_tiles[at] = tile; /* always, unless a pass before was cut short */
+            if (at < B.n_row_tiles) B.far_tiles[at] = tile; /* always: a pass starts with a count of zero */
         }
     }
     if constexpr (CB > 0) { /* the halo rows, one per thread, and the layer's weights */
