@@ -51,7 +51,13 @@ constexpr int BT = VMHIP_HTILE;   /* rows of a half tile */
 constexpr int BH = VMHIP_HHALO;   /* halo rows staged beside them */
 constexpr int BROWS = BT + BH;    /* LDS rows per buffer */
 constexpr int NOTE = VMHIP_NOTE_WORDS;
-constexpr int SC = 32;                            /* channels of a stage */
+constexpr int C = 64, SLOTS = 7, NN = SLOTS - 1;  /* the shape: C -> C channels */
+constexpr int ROWB = C * 4;                       /* bytes of a row */
+constexpr int SC = 32, STAGES = C / SC;           /* channels of a stage, stages of a half tile */
+constexpr int CHUNKS = SLOTS * 2;                 /* steps of 16 values of a stage */
+constexpr int CBW = C / 32;                       /* waves that share a row */
+constexpr int RB = CBW;                           /* blocks of 32 rows of a wave: 128 rows over 4 / CBW waves; a stage finishes one */
+constexpr int PER = 6 * RB;                       /* matrix instructions of a step */
 constexpr int PART = BROWS * SC * 2;              /* one part of a stage's rows */
 constexpr int PLANES = 3 * PART;
 constexpr int LANDING = BROWS * SC * 4;           /* a stage's rows as they arrive */
@@ -60,26 +66,14 @@ constexpr int GROUPS = BROWS / 16 / 4;            /* groups of 16 rows that a wa
 constexpr int PIECES = 14;                        /* ... in so many pieces of side work each */
 constexpr int N_SLICES = 20;                      /* of a finished row block: 16 activations, 4 stores */
 constexpr int N_STORES = 4;
-/* slots whose weights' low parts lie in LDS, where the registers do not hold all parts */
-constexpr int low_slots(int c_in) { return c_in > 32 ? 3 : 0; }
-constexpr size_t low_bytes(int c_in, int c_out) { return size_t(low_slots(c_in)) * (c_in / 16) * (c_out > 32 ? 2 : 1) * 1024; }
-constexpr size_t x3_lds_bytes(int c_in, int c_out) { return 2 * PLANES + LANDING + 4 * NBL + 4 * NOTE * 4 + 64 * 4 + low_bytes(c_in, c_out); }
+constexpr int LOW_SLOTS = 3, LOW_FROM = SLOTS - LOW_SLOTS; /* the last slots, whose weights' low parts lie in LDS: the registers do not hold them all */
+constexpr size_t LDS_BYTES = 2 * PLANES + LANDING + 4 * NBL + 4 * NOTE * 4 + C * 4 + size_t(LOW_SLOTS) * (C / 16) * CBW * 1024;
+static_assert(NN <= VMHIP_NBL_STRIDE, "the half-tile neighbour table holds 8 entries per row");
+static_assert(STAGES == RB, "a stage finishes one row block");
+static_assert(LDS_BYTES <= 160 * 1024, "the block must fit the CU's LDS");
 
-template <int C_IN, int C_OUT, int SLOTS, int ACT>
+template <int ACT>
 __global__ __launch_bounds__(256) void vm_conv_x3_kernel(VmBatchDev B, VmLayerDev L, const float* __restrict__ in, float* __restrict__ out) {
-    constexpr int NN = SLOTS - 1;
-    constexpr int NCH = C_IN / SC;                /* stages of a half tile */
-    constexpr int CBW = (C_OUT + 31) / 32;        /* waves that share a row */
-    constexpr int RB = CBW;                       /* blocks of 32 rows of a wave: 128 rows over 4 / CBW waves */
-    constexpr int ROWB = C_IN * 4, OUTB = C_OUT * 4;
-    constexpr int CHUNKS = SLOTS * 2;             /* steps of 16 values of a stage */
-    constexpr int AHEAD = RB == 1 ? 2 : 1, NB = AHEAD + 1; /* the steps by which an operand is read before it is used */
-    constexpr int PER = 6 * RB;                   /* matrix instructions of a step */
-    constexpr int LOOK = 2 / NCH;                 /* half tiles by which the loads are ahead: two stages */
-    constexpr int LOW_FROM = SLOTS - low_slots(C_IN);
-    static_assert(NN > 0 && NN <= VMHIP_NBL_STRIDE, "the half-tile neighbour table holds 8 entries per row");
-    static_assert((NCH == 1 || NCH == 2) && CBW <= 2 && NCH == RB, "a stage finishes one row block");
-
     extern __shared__ float4 lds4[];
     char* const lds = reinterpret_cast<char*>(lds4);
     const int lane = threadIdx.x & 63;
@@ -91,7 +85,7 @@ __global__ __launch_bounds__(256) void vm_conv_x3_kernel(VmBatchDev B, VmLayerDe
     char* const nbl_lds = lds + 2 * PLANES + LANDING + wave * NBL;
     uint32_t* const slot = reinterpret_cast<uint32_t*>(lds + 2 * PLANES + LANDING + 4 * NBL) + wave * NOTE;
     float* const b_lds = reinterpret_cast<float*>(lds + 2 * PLANES + LANDING + 4 * NBL + 4 * NOTE * 4);
-    v4u* const low_lds = reinterpret_cast<v4u*>(b_lds + 64) + cb * (low_slots(C_IN) * NCH * 2 * 64) + lane;
+    v4u* const low_lds = reinterpret_cast<v4u*>(b_lds + C) + cb * (LOW_SLOTS * STAGES * 2 * 64) + lane;
 
     /* half tiles in use, and this block's share: XCD-aware (block b works for XCD b % 8 on a contiguous eighth) */
     const int n_tiles = B.active_h[B.n_frames];
@@ -102,11 +96,11 @@ __global__ __launch_bounds__(256) void vm_conv_x3_kernel(VmBatchDev B, VmLayerDe
     const int count = tile0 < t_end ? (t_end - tile0 + gx - 1) / gx : 0; /* half tiles of this block: tile0 + k * gx, k < count */
 
     /* the wave's weights: [cb][stage][slot][step][h, m, l][lane] 16 bytes each */
-    v4u w[NCH][SLOTS][2][3];
+    v4u w[STAGES][SLOTS][2][3];
     {
-        const v4u* wp = reinterpret_cast<const v4u*>(L.w_x3) + (size_t) cb * (NCH * SLOTS * 2 * 3 * 64) + lane;
+        const v4u* wp = reinterpret_cast<const v4u*>(L.w_x3) + (size_t) cb * (STAGES * SLOTS * 2 * 3 * 64) + lane;
 #pragma unroll
-        for (int c = 0; c < NCH; ++c)
+        for (int c = 0; c < STAGES; ++c)
 #pragma unroll
             for (int s = 0; s < SLOTS; ++s)
 #pragma unroll
@@ -118,12 +112,12 @@ __global__ __launch_bounds__(256) void vm_conv_x3_kernel(VmBatchDev B, VmLayerDe
                         else w[c][s][j][p] = t;
                     }
     }
-    if (threadIdx.x < 64) b_lds[threadIdx.x] = (int) threadIdx.x < C_OUT ? L.b[threadIdx.x] : 0.0f;
+    if (threadIdx.x < C) b_lds[threadIdx.x] = L.b[threadIdx.x];
     /* Every load the compiler knows of returns before the first one it does not know of is issued. The same statements say where
      * the weights live: at most 64 tuples fill the accumulation registers, from which the matrix instruction reads its operands as
      * well as from vector registers, the others stay in the vector file. No instantiation may spill (conv_bf16.hip says why). */
 #pragma unroll
-    for (int c = 0; c < NCH; ++c)
+    for (int c = 0; c < STAGES; ++c)
 #pragma unroll
         for (int s = 0; s < SLOTS; ++s)
 #pragma unroll
@@ -152,7 +146,7 @@ __global__ __launch_bounds__(256) void vm_conv_x3_kernel(VmBatchDev B, VmLayerDe
         return make_int4(__builtin_amdgcn_readfirstlane((int) d.x), __builtin_amdgcn_readfirstlane((int) d.y),
                          __builtin_amdgcn_readfirstlane((int) d.z), __builtin_amdgcn_readfirstlane((int) d.w));
     };
-    /* the wave's rows of the neighbour table of the half tile at d: 64 rows from rw * 32 RB (with one row block 32 more than it uses) */
+    /* the wave's rows of the neighbour table of the half tile at d */
     auto request_nbl = [&](const int4& d, bool live) {
         load_to_lds_b128(nbl_rsrc, lds_address(nbl_lds), live ? (uint32_t) (d.x + rw * (32 * RB) + lane) * (VMHIP_NBL_STRIDE * 2) : OOR);
     };
@@ -220,10 +214,10 @@ __global__ __launch_bounds__(256) void vm_conv_x3_kernel(VmBatchDev B, VmLayerDe
     auto tile_of = [&](int k) { return tile0 + k * gx; };
     auto walk = [&]() {
         /* ---- prologue: the first stage split, the second on its way ---- */
-        int4 d_next, d_ahead; /* half tiles k + 1 and, with one stage to a half tile, k + 2 */
+        int4 d_next; /* half tile k + 1 */
         request_note(tile_of(0), true);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        d_next = d_ahead = read_note();
+        d_next = read_note();
         {
             const Source S = source(d_next, true);
 #pragma unroll
@@ -235,20 +229,10 @@ __global__ __launch_bounds__(256) void vm_conv_x3_kernel(VmBatchDev B, VmLayerDe
 #pragma unroll
                 for (int i = 0; i < 12; ++i) split_piece(i, q, planes);
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); /* the landing has been read: it may be written again */
-            if constexpr (NCH == 2) {
 #pragma unroll
-                for (int i = 0; i < 2 * GROUPS; ++i) request_rows(i >> 1, i & 1, 1, S);
-            }
-            else {
-                request_note(tile_of(min(1, count - 1)), 1 < count);
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                d_ahead = read_note();
-                const Source S1 = source(d_ahead, 1 < count);
-#pragma unroll
-                for (int i = 0; i < 2 * GROUPS; ++i) request_rows(i >> 1, i & 1, 0, S1);
-            }
+            for (int i = 0; i < 2 * GROUPS; ++i) request_rows(i >> 1, i & 1, 1, S);
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); /* and so has the slot */
-            request_note(tile_of(min(LOOK, count - 1)), LOOK < count);
+            request_note(tile_of(min(1, count - 1)), 1 < count);
         }
 
         /* the finished sums of the half tile before, waiting for activation and store: a row block per stage */
@@ -269,11 +253,11 @@ __global__ __launch_bounds__(256) void vm_conv_x3_kernel(VmBatchDev B, VmLayerDe
             else if (i < N_SLICES) {
                 const int g = i - 16; /* two lanes write 32 bytes of a row with one instruction */
                 __builtin_amdgcn_raw_buffer_store_b128(v4u{__float_as_uint(done[rb][g * 4]), __float_as_uint(done[rb][g * 4 + 1]), __float_as_uint(done[rb][g * 4 + 2]), __float_as_uint(done[rb][g * 4 + 3])}, rs,
-                                                       g * 8 < C_OUT ? done_at[rb] + (uint32_t) (g * 32) : NOWHERE, 0, 0);
+                                                       done_at[rb] + (uint32_t) (g * 32), 0, 0);
             }
         };
         auto out_window = [&]() {
-            return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<char*>(out) + (size_t) done_first * OUTB, 0, BT * OUTB, 0x00020000);
+            return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<char*>(out) + (size_t) done_first * ROWB, 0, BT * ROWB, 0x00020000);
         };
 
         v16f big[RB], small[RB]; /* the products of the high parts; the others */
@@ -282,9 +266,9 @@ __global__ __launch_bounds__(256) void vm_conv_x3_kernel(VmBatchDev B, VmLayerDe
             uint32_t own[RB];
             bool valid[RB];
             v4u nbl[RB];
-            static_for<NCH>([&](auto stage_tag) {
+            static_for<STAGES>([&](auto stage_tag) {
                 constexpr int stage = decltype(stage_tag)::value;
-                const int at_stage = (k * NCH + stage) & 1;
+                const int at_stage = (k * STAGES + stage) & 1;
                 const char* const rows = planes + at_stage * PLANES;
                 char* const split_into = planes + (at_stage ^ 1) * PLANES;
                 /* My loads of the stage before have landed once nothing but the stores issued after them can be in flight (vector
@@ -293,10 +277,7 @@ __global__ __launch_bounds__(256) void vm_conv_x3_kernel(VmBatchDev B, VmLayerDe
                 else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N_STORES) : "memory");
                 __syncthreads(); /* everyone has split this stage's rows, and read the last of those that are split next */
                 if constexpr (stage == 0) {
-                    d_next = d_ahead;
-                    const int4 d = read_note();
-                    d_ahead = d;
-                    if constexpr (NCH == 2) d_next = d;
+                    d_next = read_note();
 #pragma unroll
                     for (int rb = 0; rb < RB; ++rb) {
                         const int own_at = (rw * RB + rb) * 32 + r32;
@@ -312,10 +293,10 @@ __global__ __launch_bounds__(256) void vm_conv_x3_kernel(VmBatchDev B, VmLayerDe
                         }
                     }
                 }
-                const Source S = source(d_ahead, k + LOOK < count);
+                const Source S = source(d_next, k + 1 < count);
                 const __amdgpu_buffer_rsrc_t rs = out_window();
 
-                v4u x[NB][RB][3];
+                v4u x[2][RB][3];
                 uint32_t at[RB]; /* where the lane's piece of the slot's row lies; the second step is an exclusive or away */
                 auto gather = [&](int c, int rb) {
                     const int s = c >> 1, j = c & 1;
@@ -324,7 +305,7 @@ __global__ __launch_bounds__(256) void vm_conv_x3_kernel(VmBatchDev B, VmLayerDe
                     if (j == 0) at[rb] = li * 64u + (((uint32_t) h ^ ((li >> 2) & 3u)) * 16u);
                     const char* const p = rows + (at[rb] ^ (uint32_t) (j * 32));
 #pragma unroll
-                    for (int t = 0; t < 3; ++t) x[c % NB][rb][t] = *reinterpret_cast<const v4u*>(p + t * PART);
+                    for (int t = 0; t < 3; ++t) x[c % 2][rb][t] = *reinterpret_cast<const v4u*>(p + t * PART);
                 };
                 /* The side work of a stage in the order it is issued: the next stage's four groups of rows are split, the stage after that
                  * is requested into the places they leave; the neighbour table of the next half tile; the note of the one that is
@@ -340,7 +321,7 @@ __global__ __launch_bounds__(256) void vm_conv_x3_kernel(VmBatchDev B, VmLayerDe
                         if constexpr (stage == 0) request_nbl(d_next, k + 1 < count);
                     }
                     else if constexpr (i == GROUPS * PIECES + 1) {
-                        if constexpr (stage == NCH - 1) request_note(tile_of(min(k + LOOK + 1, count - 1)), k + LOOK + 1 < count);
+                        if constexpr (stage == STAGES - 1) request_note(tile_of(min(k + 2, count - 1)), k + 2 < count);
                     }
                     else if constexpr (i < GROUPS * PIECES + 2 + N_SLICES) {
                         finish_slice(i - (GROUPS * PIECES + 2), stage, rs);
@@ -348,25 +329,23 @@ __global__ __launch_bounds__(256) void vm_conv_x3_kernel(VmBatchDev B, VmLayerDe
                 };
                 static_assert(CHUNKS * 6 >= GROUPS * PIECES + 2 + N_SLICES, "every item of the side work finds its place");
 #pragma unroll
-                for (int c = 0; c < AHEAD; ++c)
-#pragma unroll
-                    for (int rb = 0; rb < RB; ++rb) gather(c, rb);
+                for (int rb = 0; rb < RB; ++rb) gather(0, rb);
                 static_for<CHUNKS>([&](auto chunk) {
                     constexpr int c = decltype(chunk)::value, s = c >> 1, j = c & 1;
                     v4u low;
                     static_for<PER>([&](auto mm) {
                         constexpr int m = decltype(mm)::value, rb = m % RB, kind = m / RB;
                         const v8bf a = __builtin_bit_cast(v8bf, s >= LOW_FROM && kind == 4 ? low : w[stage][s][j][WP[kind]]);
-                        const v8bf b = __builtin_bit_cast(v8bf, x[c % NB][rb][XP[kind]]);
+                        const v8bf b = __builtin_bit_cast(v8bf, x[c % 2][rb][XP[kind]]);
                         v16f& acc = kind == 5 ? big[rb] : small[rb];
                         acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
                         __builtin_amdgcn_sched_barrier(0);
                         /* the operands of a step to come, once the low parts' registers are free */
-                        if constexpr (c + AHEAD < CHUNKS && (RB == 1 ? m == 3 : m == 6 || m == 8)) gather(c + AHEAD, RB == 1 ? 0 : (m - 6) / 2);
+                        if constexpr (c + 1 < CHUNKS && (m == 6 || m == 8)) gather(c + 1, (m - 6) / 2);
                         if constexpr (m == RB && s >= LOW_FROM) low = low_lds[((stage * (SLOTS - LOW_FROM) + s - LOW_FROM) * 2 + j) * 64];
-                        /* an item behind every matrix instruction or, of two row blocks, every second one, between those that
-                         * are followed by reads: what does not fit into an instruction's 32 cycles delays the next */
-                        if constexpr (RB == 1 || m % 2 == 1) item(std::integral_constant<int, (c * PER + m) / RB>());
+                        /* an item behind every second matrix instruction, between those that are followed by reads: what does not fit
+                         * into an instruction's 32 cycles delays the next */
+                        if constexpr (m % 2 == 1) item(std::integral_constant<int, (c * PER + m) / RB>());
                         __builtin_amdgcn_sched_barrier(0);
                     });
                 });
@@ -375,7 +354,7 @@ __global__ __launch_bounds__(256) void vm_conv_x3_kernel(VmBatchDev B, VmLayerDe
             done_first = (uint32_t) d_cur.x;
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb) {
-                done_at[rb] = valid[rb] ? own[rb] * OUTB + (uint32_t) (cb * 32 + h * 4) * 4 : NOWHERE;
+                done_at[rb] = valid[rb] ? own[rb] * ROWB + (uint32_t) (cb * 32 + h * 4) * 4 : NOWHERE;
 #pragma unroll
                 for (int v = 0; v < 16; ++v) done[rb][v] = big[rb][v] + small[rb][v];
             }
@@ -394,8 +373,8 @@ __global__ __launch_bounds__(256) void vm_conv_x3_kernel(VmBatchDev B, VmLayerDe
     __syncthreads(); /* biases and low parts are in LDS */
     if (count > 0) walk();
 
-    /* Half tiles with more halo rows than are staged (three in a hundred on dense meshes): every neighbour straight from memory, 64 (C_OUT 64)
-     * or 128 rows at a time, the operands of DEEP steps under way at once. The same instructions on the same parts in the same order as
+    /* Half tiles with more halo rows than are staged (three in a hundred on dense meshes): every neighbour straight from memory, 64 rows
+     * at a time, the operands of DEEP steps under way at once. The same instructions on the same parts in the same order as
      * above: which neighbours were staged does not show in the results. (Lanes that fetched only what was not staged, a step
      * ahead, took 40 us for a half tile.) */
     constexpr int DEEP = 6, PER_TILE = CBW;
@@ -417,12 +396,12 @@ __global__ __launch_bounds__(256) void vm_conv_x3_kernel(VmBatchDev B, VmLayerDe
         v4f ring[DEEP][2];
         auto request = [&](int c) { /* c counts the steps of all stages */
             const int stage = c / CHUNKS, s = c % CHUNKS >> 1, j = c & 1;
-            const float* const p = in + (size_t) from[s] * C_IN + stage * SC + j * 16 + h * 8;
+            const float* const p = in + (size_t) from[s] * C + stage * SC + j * 16 + h * 8;
             ring[c % DEEP][0] = *reinterpret_cast<const v4f*>(p), ring[c % DEEP][1] = *reinterpret_cast<const v4f*>(p + 4);
         };
 #pragma unroll
         for (int c = 0; c < DEEP; ++c) request(c);
-        static_for<NCH * CHUNKS>([&](auto chunk) {
+        static_for<STAGES * CHUNKS>([&](auto chunk) {
             constexpr int c = decltype(chunk)::value, stage = c / CHUNKS, s = c % CHUNKS >> 1, j = c & 1;
             v4u x[3];
 #pragma unroll
@@ -430,7 +409,7 @@ __global__ __launch_bounds__(256) void vm_conv_x3_kernel(VmBatchDev B, VmLayerDe
                 const Parts p = split_pair(ring[c % DEEP][q >> 1][(q & 1) * 2], ring[c % DEEP][q >> 1][(q & 1) * 2 + 1]);
                 x[0][q] = p.high, x[1][q] = p.middle, x[2][q] = p.low;
             }
-            if constexpr (c + DEEP < NCH * CHUNKS) request(c + DEEP);
+            if constexpr (c + DEEP < STAGES * CHUNKS) request(c + DEEP);
             v4u low = {0, 0, 0, 0};
             if constexpr (s >= LOW_FROM) low = low_lds[((stage * (SLOTS - LOW_FROM) + s - LOW_FROM) * 2 + j) * 64];
             static_for<6>([&](auto kind_tag) {
@@ -449,72 +428,57 @@ __global__ __launch_bounds__(256) void vm_conv_x3_kernel(VmBatchDev B, VmLayerDe
                     const float sum = big[g * 4 + v] + small[g * 4 + v];
                     o[v] = ACT == VMHIP_SELU ? selu(sum) : fmaxf(sum, 0.0f);
                 }
-                if (g * 8 < C_OUT) *reinterpret_cast<v4f*>(out + (size_t) (first + row) * C_OUT + cb * 32 + g * 8 + h * 4) = o;
+                *reinterpret_cast<v4f*>(out + (size_t) (first + row) * C + cb * 32 + g * 8 + h * 4) = o;
             }
         }
     }
 }
 
-template <int C_IN, int C_OUT, int SLOTS, int ACT>
+template <int ACT>
 int launch_x3(const VmBatchDev& B, const VmLayerDev& L, const float* in, float* out, hipStream_t stream) {
-    constexpr size_t lds = x3_lds_bytes(C_IN, C_OUT);
-    static_assert(lds <= 160 * 1024, "the block must fit the CU's LDS");
-    auto kernel = vm_conv_x3_kernel<C_IN, C_OUT, SLOTS, ACT>;
+    auto kernel = vm_conv_x3_kernel<ACT>;
     static std::atomic<bool> configured{false}; /* engines on several host threads may get here together */
     if (!configured) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)) != hipSuccess) {
+        if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(LDS_BYTES)) != hipSuccess) {
             (void) hipGetLastError();
             return -1;
         }
         configured = true;
     }
     /* one block of four waves per CU; the kernel reads the number of half tiles in use on the device */
-    hipLaunchKernelGGL(kernel, dim3(256), dim3(256), lds, stream, B, L, in, out);
+    hipLaunchKernelGGL(kernel, dim3(256), dim3(256), LDS_BYTES, stream, B, L, in, out);
     return 0;
 }
 
 }  // namespace
 
 /* Weight layout the kernel consumes: [column block cb][stage][slot][step j][part: h, m, l][lane = half * 32 + o][e = 0..7] bf16 of
- * W[slot * c_in + stage * 32 + j * 16 + half * 8 + e][cb * 32 + o], zero past the last column */
-size_t vm_x3_weight_bytes(int c_in, int c_out, int slots) { return size_t(slots) * c_in * ((c_out + 31) / 32 * 32) * 3 * 2; }
-void vm_x3_permute_weights(const float* w, int c_in, int c_out, int slots, void* wp) {
+ * W[slot * 64 + stage * 32 + j * 16 + half * 8 + e][cb * 32 + o] */
+size_t vm_x3_weight_bytes(void) { return size_t(SLOTS) * C * C * 3 * 2; }
+void vm_x3_permute_weights(const float* w, void* wp) {
     uint16_t* dst = reinterpret_cast<uint16_t*>(wp);
-    const int stages = c_in / 32;
-    for (int cb = 0; cb < (c_out + 31) / 32; ++cb)
-        for (int c = 0; c < stages; ++c)
-            for (int s = 0; s < slots; ++s)
+    for (int cb = 0; cb < CBW; ++cb)
+        for (int c = 0; c < STAGES; ++c)
+            for (int s = 0; s < SLOTS; ++s)
                 for (int j = 0; j < 2; ++j)
                     for (int lane = 0; lane < 64; ++lane)
                         for (int e = 0; e < 8; ++e) {
-                            const int column = cb * 32 + (lane & 31);
-                            float v = column < c_out ? w[size_t(s * c_in + c * 32 + j * 16 + (lane >> 5) * 8 + e) * c_out + column] : 0.0f;
+                            float v = w[size_t(s * C + c * SC + j * 16 + (lane >> 5) * 8 + e) * C + cb * 32 + (lane & 31)];
                             for (int p = 0; p < 3; ++p) {
                                 const uint16_t part = bf16_round(v);
-                                dst[(((((size_t(cb) * stages + c) * slots + s) * 2 + j) * 3 + p) * 64 + lane) * 8 + e] = part;
+                                dst[(((((size_t(cb) * STAGES + c) * SLOTS + s) * 2 + j) * 3 + p) * 64 + lane) * 8 + e] = part;
                                 v -= bf16_value(part);
                             }
                         }
 }
 
-#define VM_FOR_EACH_X3_SHAPE(X) X(64, 64, 7)
-
 bool vm_x3_supported(int c_in, int c_out, int slots, int activation) {
-    if (activation != VMHIP_SELU && activation != VMHIP_RELU) return false;
-#define X(CI, CO, S) if (c_in == CI && c_out == CO && slots == S) return true;
-    VM_FOR_EACH_X3_SHAPE(X)
-#undef X
-    return false;
+    return c_in == C && c_out == C && slots == SLOTS && (activation == VMHIP_SELU || activation == VMHIP_RELU);
 }
 
 int vm_launch_conv_x3(const VmBatchDev& B, const VmLayerDev& L, const float* in, float* out, hipStream_t stream, const char** kernel_name) {
     if (B.n_row_tiles <= 0) return 0;
     if (!B.row_nbl_h || !B.tile_note_h || !B.active_h || !L.w_x3 || !vm_x3_supported(L.c_in, L.c_out, L.slots, L.activation)) return -1;
     if (kernel_name) *kernel_name = vm_kernel_name("conv_x3", L.c_in, L.c_out, L.slots);
-#define X(CI, CO, S)                                       \
-    if (L.c_in == CI && L.c_out == CO && L.slots == S)     \
-        return L.activation == VMHIP_SELU ? launch_x3<CI, CO, S, VMHIP_SELU>(B, L, in, out, stream) : launch_x3<CI, CO, S, VMHIP_RELU>(B, L, in, out, stream);
-    VM_FOR_EACH_X3_SHAPE(X)
-#undef X
-    return -1;
+    return L.activation == VMHIP_SELU ? launch_x3<VMHIP_SELU>(B, L, in, out, stream) : launch_x3<VMHIP_RELU>(B, L, in, out, stream);
 }

@@ -1,5 +1,5 @@
 /*
- * conv_x3_tile.hip - fp32 graph-convolution layers with 16 or 32 input channels and up to 32 output channels on the bf16 matrix
+ * conv_x3_tile.hip - fp32 graph-convolution layers with 16 or 32 input channels and 32 output channels on the bf16 matrix
  * instructions, with every fp32 factor split into three bf16 parts (conv_x3.hip says what that computes and for which networks): neighbour
  * gather + dense + bias + activation in one kernel (reference engine/cpu/engine.hpp:213-264, apply_activation.hpp:34-84).
  *
@@ -26,26 +26,25 @@
 namespace {
 
 constexpr int NT = 512, WAVES = NT / 64;
+constexpr int C_OUT = 32, SLOTS = 7, NN = SLOTS - 1;
 constexpr int N_SLICES = 20, N_STORES = 4; /* of a wave's finished rows: 16 activations, 4 stores */
 constexpr int SLOT_WORDS = 4 + 32;         /* a wave's note of a tile: the descriptor, the halo rows it brings in */
 
 __host__ __device__ constexpr int staged_halo(int c_in) { return c_in > 16 ? VM_X3_TILE_HALO : VMHIP_HALO_MAX; }
 __host__ __device__ constexpr int staged_rows(int c_in) { return VMHIP_TILE + staged_halo(c_in); }
-__host__ __device__ constexpr int steps(int c_in, int slots) { return slots * (c_in / 16); }
-__host__ __device__ constexpr size_t tile_lds_bytes(int c_in, int slots) {
-    return size_t(staged_rows(c_in)) * c_in * (3 * 2 + 4) + WAVES * (32 * 16 + SLOT_WORDS * 4) + 32 * 4 + size_t(steps(c_in, slots)) * 1024;
+__host__ __device__ constexpr int steps(int c_in) { return SLOTS * (c_in / 16); }
+__host__ __device__ constexpr size_t tile_lds_bytes(int c_in) {
+    return size_t(staged_rows(c_in)) * c_in * (3 * 2 + 4) + WAVES * (32 * 16 + SLOT_WORDS * 4) + 32 * 4 + size_t(steps(c_in)) * 1024;
 }
 
-template <int C_IN, int C_OUT, int SLOTS, int ACT>
+template <int C_IN, int ACT>
 __global__ __launch_bounds__(NT) void vm_conv_x3_tile_kernel(VmBatchDev B, VmLayerDev L, const float* __restrict__ in, float* __restrict__ out) {
-    constexpr int NN = SLOTS - 1;
     constexpr int HALO = staged_halo(C_IN), ROWS = staged_rows(C_IN);
     constexpr int ROWB = C_IN * 4, OUTB = C_OUT * 4, PR = C_IN * 2, PART = ROWS * PR;
     constexpr int J = C_IN / 16, CHUNKS = SLOTS * J;  /* steps of 16 values per slot, and of all slots */
     constexpr int UNIT = 1024 / ROWB, LPR = 64 / UNIT; /* rows that a wave brings in with one load, lanes to a row */
     constexpr int OWN_U = VMHIP_TILE / UNIT / WAVES, HALO_U = HALO / UNIT / WAVES, UNITS = OWN_U + HALO_U;
-    constexpr int AHEAD = 1, NB = AHEAD + 1;
-    static_assert(NN > 0 && NN <= VMHIP_NBL_STRIDE && C_OUT <= 32 && (C_IN == 16 || C_IN == 32), "shapes of this kernel");
+    static_assert(NN <= VMHIP_NBL_STRIDE && (C_IN == 16 || C_IN == 32), "shapes of this kernel");
     static_assert(HALO_U * UNIT + 4 <= SLOT_WORDS && OWN_U * UNIT * WAVES == VMHIP_TILE && HALO_U * UNIT * WAVES == HALO, "the units cover the staged rows");
 
     extern __shared__ float4 lds4[];
@@ -111,12 +110,12 @@ __global__ __launch_bounds__(NT) void vm_conv_x3_tile_kernel(VmBatchDev B, VmLay
     uint32_t done_first = 0, done_at = NOWHERE;
     auto finish_slice = [&](int i, const __amdgpu_buffer_rsrc_t& rs) {
         if (i < 16) {
-            if ((i >> 2) * 8 < C_OUT) done[i] = ACT == VMHIP_SELU ? selu(done[i]) : fmaxf(done[i], 0.0f);
+            done[i] = ACT == VMHIP_SELU ? selu(done[i]) : fmaxf(done[i], 0.0f);
         }
         else if (i < N_SLICES) {
             const int g = i - 16; /* two lanes write 32 bytes of a row with one instruction */
             __builtin_amdgcn_raw_buffer_store_b128(v4u{__float_as_uint(done[g * 4]), __float_as_uint(done[g * 4 + 1]), __float_as_uint(done[g * 4 + 2]), __float_as_uint(done[g * 4 + 3])}, rs,
-                                                   g * 8 < C_OUT ? done_at + (uint32_t) (g * 32) : NOWHERE, 0, 0);
+                                                   done_at + (uint32_t) (g * 32), 0, 0);
         }
     };
     auto out_window = [&]() {
@@ -153,7 +152,7 @@ __global__ __launch_bounds__(NT) void vm_conv_x3_tile_kernel(VmBatchDev B, VmLay
         for (int c = 0; c < CHUNKS; ++c) w[c][0] = wp[(c * 3 + 0) * 64], w[c][1] = wp[(c * 3 + 1) * 64];
         for (int c = wave; c < CHUNKS; c += WAVES) low_lds[c * 64] = wp[(c * 3 + 2) * 64];
     }
-    if (threadIdx.x < 32) b_lds[threadIdx.x] = (int) threadIdx.x < C_OUT ? L.b[threadIdx.x] : 0.0f;
+    if (threadIdx.x < C_OUT) b_lds[threadIdx.x] = L.b[threadIdx.x];
     /* every load the compiler knows of has returned before the tile loop, whose waits count */
 #pragma unroll
     for (int c = 0; c < CHUNKS; ++c) asm volatile("" : "+v"(w[c][0]), "+v"(w[c][1]));
@@ -200,7 +199,7 @@ __global__ __launch_bounds__(NT) void vm_conv_x3_tile_kernel(VmBatchDev B, VmLay
             v16f big, small;
             start_sums(big, small);
             const __amdgpu_buffer_rsrc_t rs = out_window();
-            v4u x[NB][3];
+            v4u x[2][3];
             uint32_t at = 0; /* where the lane's piece of the slot's row lies; the second step is an exclusive or away */
             auto gather = [&](int c) {
                 const int s = c / J, j = c % J;
@@ -211,10 +210,9 @@ __global__ __launch_bounds__(NT) void vm_conv_x3_tile_kernel(VmBatchDev B, VmLay
                 }
                 const char* const p = planes + (at ^ (uint32_t) (j * 32));
 #pragma unroll
-                for (int t = 0; t < 3; ++t) x[c % NB][t] = *reinterpret_cast<const v4u*>(p + t * PART);
+                for (int t = 0; t < 3; ++t) x[c % 2][t] = *reinterpret_cast<const v4u*>(p + t * PART);
             };
-#pragma unroll
-            for (int c = 0; c < AHEAD; ++c) gather(c);
+            gather(0);
             static_for<CHUNKS>([&](auto chunk) {
                 constexpr int c = decltype(chunk)::value;
                 const v4u low = low_lds[c * 64];
@@ -222,9 +220,9 @@ __global__ __launch_bounds__(NT) void vm_conv_x3_tile_kernel(VmBatchDev B, VmLay
                     constexpr int kind = decltype(kind_tag)::value, m = c * 6 + kind;
                     const v8bf a = __builtin_bit_cast(v8bf, kind == 4 ? low : w[c][WP[kind] & 1]);
                     v16f& acc = kind == 5 ? big : small;
-                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, __builtin_bit_cast(v8bf, x[c % NB][XP[kind]]), acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, __builtin_bit_cast(v8bf, x[c % 2][XP[kind]]), acc, 0, 0, 0);
                     __builtin_amdgcn_sched_barrier(0);
-                    if constexpr (kind == 1 && c + AHEAD < CHUNKS) gather(c + AHEAD);
+                    if constexpr (kind == 1 && c + 1 < CHUNKS) gather(c + 1);
                     if constexpr (m % 2 == 1 && m / 2 < N_SLICES) finish_slice(m / 2, rs);
                     __builtin_amdgcn_sched_barrier(0);
                 });
@@ -285,7 +283,6 @@ __global__ __launch_bounds__(NT) void vm_conv_x3_tile_kernel(VmBatchDev B, VmLay
         if (row < in_use) {
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                if (g * 8 >= C_OUT) continue;
                 v4f o;
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
@@ -298,11 +295,11 @@ __global__ __launch_bounds__(NT) void vm_conv_x3_tile_kernel(VmBatchDev B, VmLay
     }
 }
 
-template <int C_IN, int C_OUT, int SLOTS, int ACT>
+template <int C_IN, int ACT>
 int launch_x3_tile(const VmBatchDev& B, const VmLayerDev& L, const float* in, float* out, hipStream_t stream) {
-    constexpr size_t lds = tile_lds_bytes(C_IN, SLOTS);
+    constexpr size_t lds = tile_lds_bytes(C_IN);
     static_assert(lds <= 160 * 1024, "the block must fit the CU's LDS");
-    auto kernel = vm_conv_x3_tile_kernel<C_IN, C_OUT, SLOTS, ACT>;
+    auto kernel = vm_conv_x3_tile_kernel<C_IN, ACT>;
     static std::atomic<bool> configured{false}; /* engines on several host threads may get here together */
     if (!configured) {
         if (hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)) != hipSuccess) {
@@ -319,15 +316,14 @@ int launch_x3_tile(const VmBatchDev& B, const VmLayerDev& L, const float* in, fl
 }  // namespace
 
 /* Weight layout the kernel consumes: [step c = slot * c_in / 16 + j][part: h, m, l][lane = half * 32 + o][e = 0..7] bf16 of
- * W[slot * c_in + j * 16 + half * 8 + e][o], zero past the last column */
-size_t vm_x3_tile_weight_bytes(int c_in, int, int slots) { return size_t(steps(c_in, slots)) * 3 * 64 * 16; }
-void vm_x3_tile_permute_weights(const float* w, int c_in, int c_out, int slots, void* wp) {
+ * W[slot * c_in + j * 16 + half * 8 + e][o] */
+size_t vm_x3_tile_weight_bytes(int c_in) { return size_t(steps(c_in)) * 3 * 64 * 16; }
+void vm_x3_tile_permute_weights(const float* w, int c_in, void* wp) {
     uint16_t* dst = reinterpret_cast<uint16_t*>(wp);
-    for (int c = 0; c < steps(c_in, slots); ++c)
+    for (int c = 0; c < steps(c_in); ++c)
         for (int lane = 0; lane < 64; ++lane)
             for (int e = 0; e < 8; ++e) {
-                const int o = lane & 31;
-                float v = o < c_out ? w[(size_t(c) * 16 + (lane >> 5) * 8 + e) * c_out + o] : 0.0f;
+                float v = w[(size_t(c) * 16 + (lane >> 5) * 8 + e) * C_OUT + (lane & 31)];
                 for (int p = 0; p < 3; ++p) {
                     const uint16_t part = bf16_round(v);
                     dst[((size_t(c) * 3 + p) * 64 + lane) * 8 + e] = part;
@@ -336,24 +332,15 @@ void vm_x3_tile_permute_weights(const float* w, int c_in, int c_out, int slots, 
             }
 }
 
-#define VM_FOR_EACH_X3_TILE_SHAPE(X) X(32, 32, 7) X(16, 32, 7)
-
 bool vm_x3_tile_supported(int c_in, int c_out, int slots, int activation) {
-    if (activation != VMHIP_SELU && activation != VMHIP_RELU) return false;
-#define X(CI, CO, S) if (c_in == CI && c_out == CO && slots == S) return true;
-    VM_FOR_EACH_X3_TILE_SHAPE(X)
-#undef X
-    return false;
+    return (c_in == 16 || c_in == 32) && c_out == C_OUT && slots == SLOTS && (activation == VMHIP_SELU || activation == VMHIP_RELU);
 }
 
 int vm_launch_conv_x3_tile(const VmBatchDev& B, const VmLayerDev& L, const float* in, float* out, hipStream_t stream, const char** kernel_name) {
     if (B.n_row_tiles <= 0) return 0;
     if (!B.row_nbl || !B.tile_halo || !B.tile_desc || !B.far_tiles || !L.w_x3 || !vm_x3_tile_supported(L.c_in, L.c_out, L.slots, L.activation)) return -1;
     if (kernel_name) *kernel_name = vm_kernel_name("conv_x3_tile", L.c_in, L.c_out, L.slots);
-#define X(CI, CO, S)                                       \
-    if (L.c_in == CI && L.c_out == CO && L.slots == S)     \
-        return L.activation == VMHIP_SELU ? launch_x3_tile<CI, CO, S, VMHIP_SELU>(B, L, in, out, stream) : launch_x3_tile<CI, CO, S, VMHIP_RELU>(B, L, in, out, stream);
-    VM_FOR_EACH_X3_TILE_SHAPE(X)
-#undef X
-    return -1;
+    const bool selu = L.activation == VMHIP_SELU;
+    if (L.c_in == 16) return selu ? launch_x3_tile<16, VMHIP_SELU>(B, L, in, out, stream) : launch_x3_tile<16, VMHIP_RELU>(B, L, in, out, stream);
+    return selu ? launch_x3_tile<32, VMHIP_SELU>(B, L, in, out, stream) : launch_x3_tile<32, VMHIP_RELU>(B, L, in, out, stream);
 }

@@ -134,7 +134,7 @@ struct VmBatchDev {
                            * neighbourhood kernel lists them */
     int32_t* n_far_tiles; /* how many; the last kernel of a pass leaves zero */
     int32_t halo_cap;     /* halo slots handed out per tile, <= VMHIP_HALO_MAX (smaller only to test the far path) */
-    /* the same for half tiles (null unless the engine has bf16 layers). Only half tiles with rows in use are numbered:
+    /* the same for half tiles (null unless the engine has layers for conv_bf16.hip or conv_x3.hip). Only half tiles with rows in use are numbered:
      * half tile t of frame f is number active_h[f] + t */
     int32_t* active_h;    /* [n_frames + 2] half tiles in use before each frame, their total, the entries of far_h */
     int32_t* far_h;       /* the numbers of the half tiles with neighbours that are not staged, in any order */
@@ -277,13 +277,13 @@ int vm_launch_conv_bf16(const VmBatchDev& B, const VmLayerDev& L, const void* in
 /* fp32 layers on the bf16 matrix instructions, every factor in three bf16 parts (conv_x3.hip); for finite, bounded activations; uses the
  * half-tile tables */
 bool vm_x3_supported(int c_in, int c_out, int slots, int activation);
-size_t vm_x3_weight_bytes(int c_in, int c_out, int slots);
-void vm_x3_permute_weights(const float* w, int c_in, int c_out, int slots, void* wp);
+size_t vm_x3_weight_bytes(void);
+void vm_x3_permute_weights(const float* w, void* wp);
 int vm_launch_conv_x3(const VmBatchDev& B, const VmLayerDev& L, const float* in, float* out, hipStream_t stream, const char** kernel_name);
-/* the same for 16 or 32 input and up to 32 output channels, a whole tile at a time through the tile-local tables (conv_x3_tile.hip) */
+/* the same for 16 or 32 input and 32 output channels, a whole tile at a time through the tile-local tables (conv_x3_tile.hip) */
 bool vm_x3_tile_supported(int c_in, int c_out, int slots, int activation);
-size_t vm_x3_tile_weight_bytes(int c_in, int c_out, int slots);
-void vm_x3_tile_permute_weights(const float* w, int c_in, int c_out, int slots, void* wp);
+size_t vm_x3_tile_weight_bytes(int c_in);
+void vm_x3_tile_permute_weights(const float* w, int c_in, void* wp);
 int vm_launch_conv_x3_tile(const VmBatchDev& B, const VmLayerDev& L, const float* in, float* out, hipStream_t stream, const char** kernel_name);
 
 /* matrix-core variant gathering from LDS through the tile-local tables (conv_lds.hip); fp32 rows and arithmetic,
