@@ -178,3 +178,14 @@ def test_a_delivery_serves_one_fetch():
                 del block
                 block = native.pinned_empty((need,), np.uint8)  # at the same address, as a rule
             block[:] = 0xee
+
+
+def test_cpp_calls(tmp_path):
+    """tests/native/packed_fetch.cpp: announce_packed and fetch_packed_async of the C++ engine."""
+    import os
+    import subprocess
+    root, lib_dir, exe = os.path.dirname(os.path.dirname(os.path.abspath(__file__))), os.path.dirname(native.HIP_LIB), str(tmp_path / "packed_fetch")
+    subprocess.run(["g++", "-std=c++14", "-O1", "-Wall", "-Wextra", "-Werror", "-I" + os.path.join(root, "visualmesh_amd", "cpp"), "-I" + os.path.join(root, "include"),
+                    os.path.join(root, "tests", "native", "packed_fetch.cpp"), "-L" + lib_dir, "-lvisualmesh_hip", "-Wl,-rpath," + lib_dir, "-pthread", "-o", exe], check=True)
+    out = subprocess.run([exe], capture_output=True, text=True, timeout=120)
+    assert out.returncode == 0 and out.stdout.strip() == "ok", out.stdout + out.stderr
