@@ -249,7 +249,8 @@ int vmhip_batch_fetch_packed_async(vmhip_batch* batch, void* block, size_t bytes
  * final long before the classifications, copied there while its layers work; a packed fetch into that block then brings the classifications
  * only. The announcement holds for one run, and that run may write to the block: `block` (page-locked memory from vmhip_host_alloc, at least
  * as large as that fetch will need) stays alive and unused by the caller until vmhip_batch_fetch_wait of a packed fetch, or until the
- * announcement is withdrawn with a NULL block, which waits for the copy. A block that is too small or not page-locked, and a
+ * announcement is withdrawn with a NULL block, which waits for the copy. The copy is queued by vmhip_batch_run or, after
+ * vmhip_batch_run_async, by vmhip_batch_wait, as soon as the counts of visible nodes are known: a caller that waits late has it late. A block that is too small or not page-locked, and a
  * fetch into another block or of another kind, are no errors: everything is then fetched as without an announcement.
  * vmhip_batch_delivered: the block that the last completed run has written to and that no packed fetch has followed, or NULL; a further fetch
  * of the same run brings everything, whatever has become of the block. No counterpart in the reference. */

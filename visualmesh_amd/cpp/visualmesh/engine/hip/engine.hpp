@@ -669,8 +669,9 @@ namespace engine {
             }
             /// The host side of the path: the mesh's lookup, flattened for the C ABI. Touches nothing but `fd`. `candidates`: for a call that
             /// returns results only, whose device pass tests every node against the screen; the nodes that the lookup would have
-            /// projected on the host are left to it. The whole call, before / so, in us: a projection of 9 000 nodes 300 / 120, 320x256 137 / 120, 1280x1024
-            /// 428 / 395, a Bayer frame on a mesh of 500 000 nodes 768 / 650 (with the cones projected only where it decides, and no wait in the stage).
+            /// projected on the host are left to it. The whole call, before / so, in us, together with the cones projected only where that decides
+            /// and with no wait in the stage: a projection of 9 000 nodes 302 / 122, 320x256 138 / 122, a Bayer frame on a mesh of 500 000 nodes
+            /// 773 / 654; a 1280x1024 frame 430 / 405, which is within what runs differ by.
             template <template <typename> class Model>
             static void find_ranges(const Mesh<Scalar, Model>& mesh, const mat4<Scalar>& Hoc, const Lens<Scalar>& lens, FrameData& fd, bool candidates) {
 #if defined(VISUALMESH_MESH_HAS_CONE_TREE)

@@ -36,9 +36,9 @@
  * Half tiles with more than 128 halo rows are computed again from memory at the end of the kernel, with the same parts, instructions and
  * order, so that it does not show in the results which rows were staged.
  *
- * What bounds it: power. 60 % of the cycles are matrix instructions, at 1.6 GHz; with nothing but such instructions on data like
- * this the chip runs at 1.7 (1.56 PFLOP/s; 2.0 on zeros, 2.2 GHz). 1.85 million rows: 900 us as fp32 products, 555 so, 413 by the instructions
- * alone. By size, a network 3-64-64-4 on fp32 products / so, us a pass: 4 000 rows 86 / 70, 36 000 99 / 94, 65 000 113 / 107, 130 000
+ * What bounds it: the matrix pipe at the clock that power leaves it. It is busy for 65 % of the cycles, which pass at 1.7 GHz where
+ * kernels bound by memory run at 2.4 and those of fp32 products at 2.2. A launch by rocprofv3's trace, fp32 products / so: 29.1 million
+ * rows 13.5 / 8.7 ms, 1.85 million 924 / 559 us. By size, a network 3-64-64-4 on fp32 products / so, us a pass: 4 000 rows 86 / 70, 36 000 99 / 94, 65 000 113 / 107, 130 000
  * 155 / 134, 520 000 429 / 331; with three such layers 162 / 97, 191 / 154, 212 / 173, 311 / 236, 937 / 634.
  */
 #include <atomic>

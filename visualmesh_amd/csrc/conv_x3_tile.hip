@@ -11,10 +11,11 @@
  * of side work between the matrix instructions of the one after. The two waves of a SIMD fill each other's gaps; the splitting (a sixth
  * of a tile's time) is not overlapped, there being no room for a second set of planes.
  *
- * What bounds it: power, as in conv_x3.hip. Half of the cycles are matrix instructions, at 1.6 GHz where the fp32 kernels run at 2.1. 1.06
- * million rows, as fp32 products / so: 32 -> 32 154 / 117 us by events, 16 -> 32 95 / 73 (32 -> 16 95 / 110 and 16 -> 16, 71 000 rows,
- * 9.2 / 10.8, where half of the columns are padding, stay with the fp32 instructions); sixteen frames' pass through 4-16-32-32-32-32-32-16-3
- * 824 -> 708 us. Distance of that network's probabilities from float64: 9.1e-7 -> 4.9e-7 (relative 2-norm).
+ * What bounds it: a tile's phases one after the other. By counters the matrix pipe is busy for 36 % of the cycles at 32 -> 32 and 28 % at 16 -> 32,
+ * the clock is 2.1 to 2.3 GHz and the 291 MB of a 32 -> 32 launch move at 2.8 TB/s: neither the pipe nor memory is at its limit. 1.05
+ * million rows by rocprofv3's trace, fp32 products / so: 32 -> 32 132 / 102 us, 16 -> 32 80 / 62; by events 32 -> 16 95 / 110 and
+ * 16 -> 16, 71 000 rows, 9.2 / 10.8, where half of the columns are padding: they stay with the fp32 instructions. Sixteen frames' pass
+ * through 4-16-32-32-32-32-32-16-3: 814 -> 686 us. Distance of that network's probabilities from float64: 4.0e-7 -> 2.1e-7 (root mean square).
  *
  * A tile with more than 192 halo rows, for which there is no room at 32 channels (the neighbourhood kernel lists them), is computed
  * from memory at the end, with the same parts, instructions and order: which rows were staged does not show in the results.
