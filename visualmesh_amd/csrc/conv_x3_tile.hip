@@ -11,7 +11,7 @@
  * of side work between the matrix instructions of the one after. The two waves of a SIMD fill each other's gaps; the splitting (a sixth
  * of a tile's time) is not overlapped, there being no room for a second set of planes.
  *
- * What bounds it: a tile's phases one after the other. By counters the matrix pipe is busy for 36 % of the cycles at 32 -> 32 and 28 % at 16 -> 32,
+ * What bounds it: a tile's phases one after the other. By counters the matrix pipe is busy for 37 % of the cycles at 32 -> 32 and 28 % at 16 -> 32,
  * the clock is 2.1 to 2.3 GHz and the 291 MB of a 32 -> 32 launch move at 2.8 TB/s: neither the pipe nor memory is at its limit. 1.05
  * million rows by rocprofv3's trace, fp32 products / so: 32 -> 32 132 / 102 us, 16 -> 32 80 / 62; by events 32 -> 16 95 / 110 and
  * 16 -> 16, 71 000 rows, 9.2 / 10.8, where half of the columns are padding: they stay with the fp32 instructions. Sixteen frames' pass
