@@ -541,6 +541,8 @@ namespace engine {
             size_t cached_meshes() const { return meshes_.size(); }
 
         private:
+            /// Engines with bf16 layers refuse frames of so many candidates (32-bit byte offsets into a frame's rows).
+            static constexpr int32_t MOST_CANDIDATES = (1 << 24) - 1;
             struct FlatLayer {
                 int32_t n_in, n_out, activation;
                 std::vector<float> weights, biases;
@@ -667,6 +669,11 @@ namespace engine {
             static size_t projection_bytes(const FrameData& fd) {
                 return size_t(fd.candidates) * (sizeof(std::array<Scalar, 2>) + sizeof(int32_t) + sizeof(std::array<int32_t, N>));
             }
+            static int32_t count(const std::vector<std::pair<int, int>>& ranges) {
+                int32_t n = 0;
+                for (const auto& r : ranges) n += r.second - r.first;
+                return n;
+            }
             /// The host side of the path: the mesh's lookup, flattened for the C ABI. Touches nothing but `fd`. `candidates`: for a call that
             /// returns results only, whose device pass tests every node against the screen; the nodes that the lookup would have
             /// projected on the host are left to it. The whole call, before / so, in us, together with the cones projected only where that decides
@@ -676,7 +683,11 @@ namespace engine {
             static void find_ranges(const Mesh<Scalar, Model>& mesh, const mat4<Scalar>& Hoc, const Lens<Scalar>& lens, FrameData& fd, bool candidates) {
 #if defined(VISUALMESH_MESH_HAS_CONE_TREE)
                 std::vector<std::pair<int, int>> untested;
-                const auto ranges = candidates ? mesh.lookup_candidates(Hoc, lens, untested) : mesh.lookup(Hoc, lens);
+                auto ranges = candidates ? mesh.lookup_candidates(Hoc, lens, untested) : mesh.lookup(Hoc, lens);
+                if (count(ranges) >= MOST_CANDIDATES && !untested.empty()) { /* perhaps more than an engine takes: the lookup's own nodes */
+                    untested.clear();
+                    ranges = mesh.lookup(Hoc, lens);
+                }
                 fd.untested.resize(untested.size() * 2);
                 for (size_t i = 0; i < untested.size(); ++i) fd.untested[2 * i] = untested[i].first, fd.untested[2 * i + 1] = untested[i].second;
 #else
@@ -684,12 +695,8 @@ namespace engine {
                 const auto ranges = mesh.lookup(Hoc, lens);
 #endif
                 fd.ranges.resize(ranges.size() * 2);
-                fd.candidates = 0;
-                for (size_t i = 0; i < ranges.size(); ++i) {
-                    fd.ranges[2 * i] = ranges[i].first;
-                    fd.ranges[2 * i + 1] = ranges[i].second;
-                    fd.candidates += ranges[i].second - ranges[i].first;
-                }
+                for (size_t i = 0; i < ranges.size(); ++i) fd.ranges[2 * i] = ranges[i].first, fd.ranges[2 * i + 1] = ranges[i].second;
+                fd.candidates = count(ranges);
             }
             /// Everything else about a frame whose ranges are known.
             template <template <typename> class Model>
