@@ -210,6 +210,10 @@ typedef struct vmhip_lookup_export {
 } vmhip_lookup_export;
 int vmhip_batch_export(vmhip_batch* batch, int32_t edge_type, vmhip_lookup_export* per_frame);
 int vmhip_batch_run(vmhip_batch* batch);
+/* vmhip_batch_run for a caller that goes on with vmhip_batch_fetch_held: the pass stores its results into that call's block itself, where they
+ * are no more than a few megabytes, and the fetch finds them there. The arrays of an earlier vmhip_batch_fetch_held end with this call. No
+ * counterpart in the reference. */
+int vmhip_batch_run_held(vmhip_batch* batch);
 /* The two halves of vmhip_batch_run: run_async puts the pass on the engine's stream and returns, wait blocks until it
  * is done (and settles the screen-edge decisions with the host, as run does). Between the two the caller is free,
  * e.g. to stage the next frames into a batch of another engine, whose copies then overlap this pass. Counts, fetch
@@ -246,8 +250,8 @@ int vmhip_batch_fetch_wait(vmhip_batch* batch);
 size_t vmhip_batch_fetch_packed_size(const vmhip_batch* batch);
 int vmhip_batch_fetch_packed_async(vmhip_batch* batch, void* block, size_t bytes, vmhip_result* results);
 /* Says which block the next packed fetch will be given, so that the next run can have the pixels, indices and neighbourhoods, which are
- * final long before the classifications, copied there while its layers work; a packed fetch into that block then brings the classifications
- * only. The announcement holds for one run, and that run may write to the block: `block` (page-locked memory from vmhip_host_alloc, at least
+ * final long before the classifications, copied there while its layers work, and the classifications behind them; a packed fetch into that block
+ * then has nothing left to bring. The announcement holds for one run, and that run may write to the block: `block` (page-locked memory from vmhip_host_alloc, at least
  * as large as that fetch will need) stays alive and unused by the caller until vmhip_batch_fetch_wait of a packed fetch, or until the
  * announcement is withdrawn with a NULL block, which waits for the copy. The copy is queued by vmhip_batch_run or, after
  * vmhip_batch_run_async, by vmhip_batch_wait, as soon as the counts of visible nodes are known: a caller that waits late has it late. A block that is too small or not page-locked, and a

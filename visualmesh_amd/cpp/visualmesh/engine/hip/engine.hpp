@@ -244,7 +244,7 @@ namespace engine {
             vmhip_result classify_held(const Mesh<Scalar, Model>& mesh, const mat4<Scalar>& Hoc, const Lens<Scalar>& lens,
                                        const void* image, const uint32_t& format, size_t most = std::numeric_limits<size_t>::max()) const {
                 stage_frames(std::vector<Frame<Model>>(1, Frame<Model>{&mesh, Hoc, lens, image, format}), false, true);
-                run();
+                run_held();
                 vmhip_result r{};
                 if (packed_size() > most) r.n_visible = visible_counts()[0];
                 else throw_on_error(vmhip_batch_fetch_held(batch_, &r));
@@ -262,8 +262,8 @@ namespace engine {
             /// Classify a batch of independent frames in one pass over the device.
             template <template <typename> class Model>
             std::vector<ClassifiedMesh<Scalar, Model<Scalar>::N_NEIGHBOURS>> classify(const std::vector<Frame<Model>>& frames) const {
-                stage_frames(frames, false, true); /* run() returns with the images read */
-                run();
+                stage_frames(frames, false, true); /* run_held() returns with the images read */
+                run_held();
                 return fetch<Model>();
             }
 
@@ -331,6 +331,10 @@ namespace engine {
             /// Run the staged frames on the device and wait; may be called repeatedly.
             void run() const {
                 if (batch_ && !staged_.empty()) throw_on_error(vmhip_batch_run(batch_));
+            }
+            /// The same ahead of fetch() and nothing else: the pass stores small results into the block that fetch() copies them from.
+            void run_held() const {
+                if (batch_ && !staged_.empty()) throw_on_error(vmhip_batch_run_held(batch_));
             }
             /// The same in two halves: the pass runs while the caller does something else (staging the next frames on
             /// a second engine, for one), and wait() blocks until it is done. fetch(), detect() and visible_counts()

@@ -265,8 +265,55 @@ __global__ __launch_bounds__(256) void vm_fetch_pack_kernel(const VmPackChunk* _
     }
 }
 
+__device__ __forceinline__ size_t pack_aligned(size_t bytes) { return (bytes + 255) & ~(size_t) 255; }
+/* a contiguous piece of an array, by the whole block; src and out on the 16-byte grid */
+__device__ __forceinline__ void pack_piece(const void* src, uint8_t* out, size_t bytes) {
+    const size_t vec = bytes & ~(size_t) 15;
+    for (size_t i = threadIdx.x * 16; i < vec; i += VMHIP_TILE * 16) *reinterpret_cast<uint4*>(out + i) = *reinterpret_cast<const uint4*>(static_cast<const uint8_t*>(src) + i);
+    for (size_t i = vec + threadIdx.x * 4; i < bytes; i += VMHIP_TILE * 4)
+        *reinterpret_cast<uint32_t*>(out + i) = *reinterpret_cast<const uint32_t*>(static_cast<const uint8_t*>(src) + i);
+}
+/* What frames [0, n) take of a packed block: pixels, indices and neighbourhoods, and classifications of n_classes. Every wave adds up for
+ * itself: one read per 64 frames. */
+__device__ __forceinline__ size_t packed_geometry(const VmBatchDev& B, int n) {
+    size_t at = 0;
+    for (int i = (int) (threadIdx.x & 63); i < n; i += 64) {
+        const size_t v = (size_t) B.frame_V[i], nn = (size_t) (B.uniform_nn ? B.uniform_nn : B.frames[i].nn);
+        if (v) at += pack_aligned(8 * v) + pack_aligned(4 * v) + pack_aligned(4 * (v + 1) * nn);
+    }
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) at += __shfl_xor(at, d);
+    return at;
+}
+__device__ __forceinline__ size_t packed_classes(const VmBatchDev& B, int n, int n_classes) {
+    size_t at = 0;
+    for (int i = (int) (threadIdx.x & 63); i < n; i += 64) {
+        const size_t v = (size_t) B.frame_V[i];
+        if (v) at += pack_aligned(4 * (v + 1) * (size_t) n_classes);
+    }
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) at += __shfl_xor(at, d);
+    return at;
+}
+/* a row tile's part of its frame's pixels, indices and neighbourhood; `out`: where the frame's arrays begin */
+__device__ __forceinline__ void pack_tile_geometry(const VmBatchDev& B, const VmFrame& F, int V, int row0, uint8_t* out) {
+    const size_t row = (size_t) F.row_base + row0, rows = (size_t) min(VMHIP_TILE, V - row0), nn = (size_t) F.nn;
+    const size_t nb_rows = (size_t) min(VMHIP_TILE, V + 1 - row0);
+    pack_piece(B.row_px + row, out + 8 * (size_t) row0, 8 * rows);
+    out += pack_aligned(8 * (size_t) V);
+    pack_piece(B.row_gidx + row, out + 4 * (size_t) row0, 4 * rows);
+    out += pack_aligned(4 * (size_t) V);
+    if ((size_t) B.nb_stride == nn) {
+        pack_piece(B.row_nb + row * nn, out + 4 * nn * (size_t) row0, 4 * nn * nb_rows);
+    }
+    else {
+        int32_t* const nb_out = reinterpret_cast<int32_t*>(out) + nn * (size_t) row0;
+        for (size_t i = threadIdx.x; i < nb_rows * nn; i += VMHIP_TILE) nb_out[i] = B.row_nb[(row + i / nn) * (size_t) B.nb_stride + i % nn];
+    }
+}
+
 /* vm_launch_pack_geometry: a block per row tile copies its rows of the three arrays. Where its frame's arrays go follows from the visible
- * counts of the frames before it, which every wave adds up for itself: one read per 64 frames.
+ * counts of the frames before it.
  * It stands between the neighbourhoods and the layers of a pass so that the copy over the bus runs beside the layers: three quarters of a
  * result's bytes at four classes and six neighbours. */
 __global__ __launch_bounds__(VMHIP_TILE) void vm_pack_geometry_kernel(VmBatchDev B, uint8_t* __restrict__ dst, int32_t* __restrict__ host_counts) {
@@ -278,33 +325,65 @@ __global__ __launch_bounds__(VMHIP_TILE) void vm_pack_geometry_kernel(VmBatchDev
     const VmFrame& F = B.frames[f];
     const int V = B.frame_V[f], row0 = (tile - F.row_tile0) * VMHIP_TILE;
     if (V == 0 || row0 > V) return; /* the null row is row V of the neighbourhoods */
-    auto aligned = [](size_t bytes) { return (bytes + 255) & ~(size_t) 255; };
-    size_t at = 0;
-    for (int i = (int) (threadIdx.x & 63); i < f; i += 64) {
-        const size_t v = (size_t) B.frame_V[i], nn = (size_t) (B.uniform_nn ? B.uniform_nn : B.frames[i].nn);
-        if (v) at += aligned(8 * v) + aligned(4 * v) + aligned(4 * (v + 1) * nn);
+    pack_tile_geometry(B, F, V, row0, dst + packed_geometry(B, f));
+}
+
+/* Last kernel of a pass.
+ *
+ * Blocks [0, n_frames): what the host needs of the pass is written by the device straight into page-locked host memory
+ * (block f: the head of frame f's ambiguity list; block 0 also the counts and the convolution kernel's count of waits that
+ * ran out). A copy engine is not involved, so the few hundred bytes never queue behind another engine's 50 MB download.
+ * Block 0 then prepares the next pass: the ambiguity counters (the second half of the counts) start from zero again,
+ * and the run stamp advances, so that the stamps of this pass stop matching. (As a kernel of its own at the head of a pass
+ * this cost 16 us: the pass's second kernel waited for the host to finish queueing it.) The block that is last of them says so in a word that the host
+ * may watch: the results below are stored after that, beside what the host makes of the counts.
+ *
+ * The blocks after them, if P.parts is not zero: the pass's results on their way into the block that B.delivery names, one row tile each, laid out as
+ * in a packed fetch. The caller then has them when it has waited for the pass; gathered by a fetch of its own, they cost another launch, another
+ * wait and the host's way between the two. A call or a pass with its fetch in us, that way / so: a projection of 9 000 nodes 119 / 97, eight frames through
+ * 13 thin layers 218 / 193, one frame of configuration 2 193 / 187.
+ * Many classifications go to P.classes_packed on the device, from where one copy brings them home. Nothing is written where the block is too small:
+ * the host, which sees the same counts, then fetches. */
+__global__ __launch_bounds__(VMHIP_TILE) void vm_publish_kernel(VmBatchDev B, VmPublish P) {
+    if ((int) blockIdx.x < B.n_frames) {
+        const int f = blockIdx.x, n_counts = 2 * B.n_frames;
+        for (int t = threadIdx.x; t < P.amb_head; t += VMHIP_TILE) P.host_amb[(size_t) f * P.amb_head + t] = B.amb_list[(size_t) f * VMHIP_AMB_CAP + t];
+        if (f == 0) {
+            for (int t = threadIdx.x; t < n_counts; t += VMHIP_TILE) {
+                P.host_counts[t] = B.frame_V[t];
+                if (t >= B.n_frames) B.frame_V[t] = 0; /* the ambiguity counts lie behind the visible ones */
+            }
+            if (threadIdx.x == 0) {
+                *P.host_timeouts = P.timeouts ? *P.timeouts : 0u;
+                *B.epoch += 1;
+                *B.n_far_tiles = 0;
+            }
+        }
+        __threadfence_system();
+        __syncthreads();
+        if (threadIdx.x == 0 && atomicAdd(B.published, 1u) + 1u == (uint32_t) B.n_frames) {
+            *B.published = 0u;
+            __threadfence_system();
+            __hip_atomic_store(P.host_serial, B.delivery->serial, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+        return;
     }
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) at += __shfl_xor(at, d);
-    const size_t row = (size_t) F.row_base + row0, rows = (size_t) min(VMHIP_TILE, V - row0), nn = (size_t) F.nn;
-    const size_t nb_rows = (size_t) min(VMHIP_TILE, V + 1 - row0);
-    auto copy = [&](const void* src, uint8_t* out, size_t bytes) {
-        const size_t vec = bytes & ~(size_t) 15;
-        for (size_t i = threadIdx.x * 16; i < vec; i += VMHIP_TILE * 16) *reinterpret_cast<uint4*>(out + i) = *reinterpret_cast<const uint4*>(static_cast<const uint8_t*>(src) + i);
-        for (size_t i = vec + threadIdx.x * 4; i < bytes; i += VMHIP_TILE * 4)
-            *reinterpret_cast<uint32_t*>(out + i) = *reinterpret_cast<const uint32_t*>(static_cast<const uint8_t*>(src) + i);
-    };
-    uint8_t* out = dst + at;
-    copy(B.row_px + row, out + 8 * (size_t) row0, 8 * rows);
-    out += aligned(8 * (size_t) V);
-    copy(B.row_gidx + row, out + 4 * (size_t) row0, 4 * rows);
-    out += aligned(4 * (size_t) V);
-    if ((size_t) B.nb_stride == nn) {
-        copy(B.row_nb + row * nn, out + 4 * nn * (size_t) row0, 4 * nn * nb_rows);
-    }
-    else {
-        int32_t* const nb_out = reinterpret_cast<int32_t*>(out) + nn * (size_t) row0;
-        for (size_t i = threadIdx.x; i < nb_rows * nn; i += VMHIP_TILE) nb_out[i] = B.row_nb[(row + i / nn) * (size_t) B.nb_stride + i % nn];
+    const int tile = (int) blockIdx.x - B.n_frames;
+    if (tile >= vm_row_tiles(B)) return;
+    const int f = B.row_tile_frame[tile];
+    const VmFrame& F = B.frames[f];
+    const int V = B.frame_V[f], row0 = (tile - F.row_tile0) * VMHIP_TILE;
+    if (V == 0 || row0 > V) return;
+    const VmDelivery to = *B.delivery;
+    if (!to.block) return;
+    const size_t geometry = packed_geometry(B, B.n_frames), classes = P.classes ? packed_classes(B, B.n_frames, P.n_classes) : 0;
+    if (geometry + classes > to.bytes) return;
+    if (P.parts & VM_DELIVER_GEOMETRY) pack_tile_geometry(B, F, V, row0, to.block + packed_geometry(B, f));
+    if (P.classes && (P.parts & VM_DELIVER_CLASSES)) {
+        uint8_t* const base = P.classes_packed ? P.classes_packed : to.block + geometry;
+        const size_t row_bytes = 4 * (size_t) P.n_classes;
+        pack_piece(P.classes + ((size_t) F.row_base + row0) * P.n_classes, base + packed_classes(B, f, P.n_classes) + row_bytes * row0,
+                   row_bytes * (size_t) min(VMHIP_TILE, V + 1 - row0));
     }
 }
 
@@ -313,6 +392,11 @@ __global__ __launch_bounds__(VMHIP_TILE) void vm_pack_geometry_kernel(VmBatchDev
 void vm_launch_pack_geometry(const VmBatchDev& B, void* dst, int32_t* host_counts, hipStream_t stream) {
     if (B.n_row_tiles <= 0) return;
     hipLaunchKernelGGL(vm_pack_geometry_kernel, dim3(B.n_row_tiles), dim3(VMHIP_TILE), 0, stream, B, static_cast<uint8_t*>(dst), host_counts);
+}
+
+void vm_launch_publish(const VmBatchDev& B, const VmPublish& P, hipStream_t stream) {
+    const int tiles = P.parts ? B.n_row_tiles : 0;
+    hipLaunchKernelGGL(vm_publish_kernel, dim3((B.n_frames > 0 ? B.n_frames : 1) + tiles), dim3(VMHIP_TILE), 0, stream, B, P);
 }
 
 void vm_launch_fetch_pack(const VmPackChunk* chunks, int n_chunks, void* dst, hipStream_t stream) {

@@ -15,8 +15,6 @@
  *                            ascending local row; writes pixel, global index, reverse lookup stamp and the
  *                            sampled 4-channel input row; the frame's last tile writes V and the null row
  *   vm_neighbourhood_kernel  row space: neighbour table through the stamped reverse lookup
- *   vm_publish_kernel        (after the network) counts and ambiguity lists into page-locked host memory; clears the
- *                            ambiguity counters and advances the run stamp for the next pass
  */
 #include "vmhip_internal.h"
 
@@ -200,30 +198,6 @@ __global__ __launch_bounds__(256) void vm_stage_kernel(const void* __restrict__ 
     copy(b_src, b_dst, b_bytes);
     for (size_t i = first; i < n_clear; i += step) clear0[i] = clear1[i] = make_uint2(0u, 0u);
     for (size_t i = first; i < n_clear2; i += step) clear2[i] = make_uint2(0u, 0u);
-}
-
-/* Last kernel of a pass. What the host needs of the pass is written by the device straight into page-locked host memory
- * (block f: the head of frame f's ambiguity list; block 0 also the counts and the convolution kernel's count of waits that
- * ran out). A copy engine is not involved, so the few hundred bytes never queue behind another engine's 50 MB download.
- * Block 0 then prepares the next pass: the ambiguity counters (the second half of the counts) start from zero again,
- * and the run stamp advances, so that the stamps of this pass stop matching. (As a kernel of its own at the head of a pass
- * this cost 16 us: the pass's second kernel waited for the host to finish queueing it.) */
-__global__ __launch_bounds__(64) void vm_publish_kernel(int32_t* __restrict__ counts, int n_counts, const int2* __restrict__ amb_list, int amb_stride,
-                                                        int amb_head, const unsigned int* __restrict__ timeouts, uint32_t* __restrict__ epoch, int32_t* __restrict__ n_far_tiles,
-                                                        int32_t* host_counts, int2* host_amb, uint32_t* host_timeouts) {
-    const int f = blockIdx.x;
-    for (int t = threadIdx.x; t < amb_head; t += 64) host_amb[(size_t) f * amb_head + t] = amb_list[(size_t) f * amb_stride + t];
-    if (f == 0) {
-        for (int t = threadIdx.x; t < n_counts; t += 64) {
-            host_counts[t] = counts[t];
-            if (t >= n_counts / 2) counts[t] = 0;
-        }
-        if (threadIdx.x == 0) {
-            *host_timeouts = timeouts ? *timeouts : 0u;
-            *epoch += 1;
-            *n_far_tiles = 0;
-        }
-    }
 }
 
 /* ---- lookup on the device: the host's walk of the cone tree (cpp/visualmesh/detail/cone_tree.hpp, itself after the
@@ -471,6 +445,8 @@ __global__ __launch_bounds__(VMHIP_TILE) void vm_lookup_export_kernel(VmBatchDev
 __global__ __launch_bounds__(VMHIP_TILE) void vm_project_kernel(VmBatchDev B) {
     __shared__ int wave_count[VMHIP_TILE / 64];
     const int tile = blockIdx.x;
+    /* where the pass's results go is the host's to change from pass to pass: fetched over the bus once, here, not by every block of the last kernel */
+    if (tile == 0 && threadIdx.x == 0 && B.delivery) *B.delivery = *B.order;
     if (tile >= vm_cand_tiles(B)) return; /* the grid may be sized for more tiles than the staged batch has */
     int f, tile_range = -1;
     if (B.cand_tile_info) {
@@ -1086,11 +1062,6 @@ void vm_launch_stage(const void* a_src, void* a_dst, size_t a_bytes, const void*
                        static_cast<uint2*>(clear0), static_cast<uint2*>(clear1), n_clear, static_cast<uint2*>(clear2), clear2_bytes / 8);
 }
 
-void vm_launch_publish(int32_t* counts, int n_counts, const int2* amb_list, int amb_stride, int amb_head, int n_frames, const unsigned int* timeouts, uint32_t* epoch, int32_t* n_far_tiles,
-                       int32_t* host_counts, int2* host_amb, uint32_t* host_timeouts, hipStream_t stream) {
-    hipLaunchKernelGGL(vm_publish_kernel, dim3(n_frames > 0 ? n_frames : 1), dim3(64), 0, stream, counts, n_counts, amb_list, amb_stride, amb_head, timeouts, epoch, n_far_tiles,
-                       host_counts, host_amb, host_timeouts);
-}
 void vm_launch_project(const VmBatchDev& B, hipStream_t stream) {
     if (B.n_cand_tiles > 0) hipLaunchKernelGGL(vm_project_kernel, dim3(B.n_cand_tiles), dim3(VMHIP_TILE), 0, stream, B);
 }

@@ -97,6 +97,15 @@ struct VmBatchLive {
     int32_t n_cand_tiles, n_row_tiles;
 };
 
+/* Where the results of a pass go while it runs (detect.hip: vm_publish_kernel): a page-locked block, laid out as in a packed fetch. The host
+ * writes it beside the landing area before each pass, whose first kernel brings it to the device, so that a captured pass may be given
+ * another block every time. */
+struct VmDelivery {
+    uint8_t* block;       /* null: nowhere */
+    uint64_t bytes;
+    uint32_t serial;      /* the pass's number */
+};
+
 struct VmBatchDev {
     const VmFrame* frames;
     int32_t n_frames;
@@ -140,6 +149,9 @@ struct VmBatchDev {
     int32_t* far_h;       /* the numbers of the half tiles with neighbours that are not staged, in any order */
     uint16_t* row_nbl_h;  /* [rows][VMHIP_NBL_STRIDE]: 0..127 own half tile, 128+h halo slot h, VMHIP_NBL_FAR not staged */
     uint32_t* tile_note_h; /* [half tiles in use][VMHIP_NOTE_WORDS] */
+    const VmDelivery* order; /* page-locked host memory; null beside a null delivery */
+    VmDelivery* delivery;    /* the pass's copy of it; null: the batch's passes deliver nothing */
+    uint32_t* published;     /* how many frames the pass's last kernel has published; it leaves zero */
     unsigned int* flow_timeouts; /* the batch's count of waits of the barrier-free kernel that ran out of polls (0 in a correct run) */
     /* edge guard: a candidate closer than amb_eps pixels to a screen edge is listed for the host's re-decision.
      * px_error is 0 outside tests: added to both pixel coordinates, it stands for a device whose lens arithmetic
@@ -242,10 +254,22 @@ void vm_launch_libm(int which, const float* x, float* y, int n, hipStream_t stre
 void vm_launch_copy_probe(const void* src, void* dst, size_t bytes, hipStream_t stream);
 /* rows: a multiple of 64; bytes per row: multiples of 4 (64 rows are whole 16-byte pieces then) */
 void vm_launch_stream_probe(const void* src, void* dst, size_t rows, int read_bytes_per_row, int write_bytes_per_row, hipStream_t stream);
-/* counts[n_counts], the first amb_head entries of every frame's ambiguity list and the timeout count, stored by the device
- * into page-locked host memory (device-visible pointers) */
-void vm_launch_publish(int32_t* counts, int n_counts, const int2* amb_list, int amb_stride, int amb_head, int n_frames, const unsigned int* timeouts, uint32_t* epoch, int32_t* n_far_tiles,
-                       int32_t* host_counts, int2* host_amb, uint32_t* host_timeouts, hipStream_t stream);
+/* The pass's last kernel (detect.hip): visible and ambiguity counts, the first amb_head entries of every frame's ambiguity list and the timeout count,
+ * stored by the device into page-locked host memory (device-visible pointers); `parts` of the results into the block of B.delivery. */
+enum { VM_DELIVER_GEOMETRY = 1, VM_DELIVER_CLASSES = 2 };
+struct VmPublish {
+    int32_t amb_head;
+    int32_t parts;            /* VM_DELIVER_*: at most VM_GEOMETRY_FRAMES frames, staged with their tile tables */
+    const unsigned int* timeouts;
+    int32_t* host_counts;
+    int2* host_amb;
+    uint32_t* host_timeouts;
+    uint32_t* host_serial;    /* gets VmDelivery::serial when everything above is there */
+    const float* classes;     /* [rows][n_classes], or null */
+    int32_t n_classes;
+    uint8_t* classes_packed;  /* device memory with room for all classifications, to leave them there; null: into the block */
+};
+void vm_launch_publish(const VmBatchDev& B, const VmPublish& P, hipStream_t stream);
 void vm_launch_project(const VmBatchDev& B, hipStream_t stream);
 void vm_launch_compact(const VmBatchDev& B, float* feat, int classify, hipStream_t stream);
 void vm_launch_neighbourhood(const VmBatchDev& B, hipStream_t stream); /* also the tile-local tables if B.row_nbl */

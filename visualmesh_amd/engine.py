@@ -298,20 +298,13 @@ class Engine:
         n_out = self.network.n_out
         out = []
         base = block.ctypes.data
-        for i in range(n):
-            V = raw[i].n_visible
-            nn = self._staged[i].n_neighbours
+        for (_, V, px, gidx, nb, cls), m in zip(np.frombuffer(raw, native.RESULT_DTYPE).tolist(), self._staged):
+            nn = m.n_neighbours
             if V == 0:
                 out.append(dict(px=np.zeros((0, 2), np.float32), nb=np.zeros((0, nn), np.int32), gidx=np.zeros(0, np.int32), cls=np.zeros((0, n_out), np.float32)))
                 continue
-
-            def view(pointer, count, dtype, shape):
-                at = C.cast(pointer, C.c_void_p).value - base
-                return block[at:at + count * 4].view(dtype).reshape(shape)
-
-            out.append(dict(px=view(raw[i].pixel_coordinates, 2 * V, np.float32, (V, 2)), gidx=view(raw[i].global_indices, V, np.int32, (V,)),
-                            nb=view(raw[i].neighbourhood, (V + 1) * nn, np.int32, (V + 1, nn)),
-                            cls=view(raw[i].classifications, (V + 1) * n_out, np.float32, (V + 1, n_out))))
+            out.append(dict(px=np.ndarray((V, 2), np.float32, block, px - base), gidx=np.ndarray((V,), np.int32, block, gidx - base),
+                            nb=np.ndarray((V + 1, nn), np.int32, block, nb - base), cls=np.ndarray((V + 1, n_out), np.float32, block, cls - base)))
         self._raw_results = raw
         if wait:
             self.fetch_wait()
