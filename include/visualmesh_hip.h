@@ -210,10 +210,6 @@ typedef struct vmhip_lookup_export {
 } vmhip_lookup_export;
 int vmhip_batch_export(vmhip_batch* batch, int32_t edge_type, vmhip_lookup_export* per_frame);
 int vmhip_batch_run(vmhip_batch* batch);
-/* vmhip_batch_run for a caller that goes on with vmhip_batch_fetch_held: the pass stores its results into that call's block itself, where they
- * are no more than a few megabytes, and the fetch finds them there. The arrays of an earlier vmhip_batch_fetch_held end with this call. No
- * counterpart in the reference. */
-int vmhip_batch_run_held(vmhip_batch* batch);
 /* The two halves of vmhip_batch_run: run_async puts the pass on the engine's stream and returns, wait blocks until it
  * is done (and settles the screen-edge decisions with the host, as run does). Between the two the caller is free,
  * e.g. to stage the next frames into a batch of another engine, whose copies then overlap this pass. Counts, fetch
@@ -268,6 +264,13 @@ void* vmhip_batch_delivered(const vmhip_batch* batch);
  * and given back by the next one: a caller that has arrays of its own uses vmhip_batch_fetch there. No counterpart in the reference. */
 #define VMHIP_HELD_MOST ((size_t) 64 << 20)
 int vmhip_batch_fetch_held(vmhip_batch* batch, vmhip_result* results);
+/* Stage, run and fetch_held of one call, whose caller copies the results away: classify_begin returns when pixels, indices and neighbourhoods are there
+ * (results[i] as from vmhip_batch_fetch_held) while the network still runs, classify_end when the classifications are too. Nothing of the former needs an image, so
+ * that the images cross the bus beside it, and the copies of a caller who makes them between the two cost no time of their own. The images stay as
+ * they are until classify_end has returned; between the two calls the batch is used for nothing else. More than VMHIP_HELD_MOST bytes of results stay on the
+ * device, as after vmhip_batch_run: n_visible is set, the pointers are NULL. No counterpart in the reference. */
+int vmhip_batch_classify_begin(vmhip_batch* batch, const vmhip_frame* frames, int32_t n_frames, vmhip_result* results);
+int vmhip_batch_classify_end(vmhip_batch* batch);
 /* vmhip_project with its results in a block that belongs to the engine, until the engine's next vmhip_project_held */
 int vmhip_project_held(vmhip_engine* engine, const vmhip_frame* frame, vmhip_result* result);
 

@@ -237,18 +237,18 @@ namespace engine {
                 std::vector<Frame<Model>> one(1, Frame<Model>{&mesh, Hoc, lens, image, format});
                 return std::move(classify(one)[0]);
             }
-            /// The same with the results left in a block of the engine's (see vmhip_batch_fetch_held), which its next fetch()
-            /// or classification overwrites: n_visible rows, and null pointers if that is zero. More than `most` bytes of results
-            /// stay on the device, as after run(): n_visible is set, the pointers are null.
+            /// The same in two halves, with the results left in a block of the engine's (see vmhip_batch_classify_begin), which its next fetch()
+            /// or classification overwrites: n_visible rows, and null pointers if that is zero. What classify_begin() returns is valid at once but for
+            /// the classifications, which are there when classify_end() has returned; the image must stay as it is until then. More than VMHIP_HELD_MOST
+            /// bytes of results stay on the device, as after run(): n_visible is set, the pointers are null.
             template <template <typename> class Model>
-            vmhip_result classify_held(const Mesh<Scalar, Model>& mesh, const mat4<Scalar>& Hoc, const Lens<Scalar>& lens,
-                                       const void* image, const uint32_t& format, size_t most = std::numeric_limits<size_t>::max()) const {
-                stage_frames(std::vector<Frame<Model>>(1, Frame<Model>{&mesh, Hoc, lens, image, format}), false, true);
-                run_held();
-                vmhip_result r{};
-                if (packed_size() > most) r.n_visible = visible_counts()[0];
-                else throw_on_error(vmhip_batch_fetch_held(batch_, &r));
-                return r;
+            vmhip_result classify_begin(const Mesh<Scalar, Model>& mesh, const mat4<Scalar>& Hoc, const Lens<Scalar>& lens, const void* image, const uint32_t& format) const {
+                std::vector<vmhip_result> r(1);
+                stage_frames(std::vector<Frame<Model>>(1, Frame<Model>{&mesh, Hoc, lens, image, format}), Stage::CALL, &r);
+                return r[0];
+            }
+            void classify_end() const {
+                if (batch_) throw_on_error(vmhip_batch_classify_end(batch_));
             }
             template <template <typename> class Model>
             ClassifiedMesh<Scalar, Model<Scalar>::N_NEIGHBOURS> operator()(const VisualMesh<Scalar, Model>& mesh,
@@ -262,27 +262,53 @@ namespace engine {
             /// Classify a batch of independent frames in one pass over the device.
             template <template <typename> class Model>
             std::vector<ClassifiedMesh<Scalar, Model<Scalar>::N_NEIGHBOURS>> classify(const std::vector<Frame<Model>>& frames) const {
-                stage_frames(frames, false, true); /* run_held() returns with the images read */
-                run_held();
-                return fetch<Model>();
+                constexpr int N = Model<Scalar>::N_NEIGHBOURS;
+                std::vector<ClassifiedMesh<Scalar, N>> out(frames.size());
+                if (frames.empty()) {
+                    stage_frames(frames, Stage::ASYNC);
+                    return out;
+                }
+                std::vector<vmhip_result> results(frames.size());
+                stage_frames(frames, Stage::CALL, &results);
+                bool on_device = false;
+                try {  // the network is still at work
+                    for (size_t i = 0; i < out.size(); ++i) {
+                        if (results[i].n_visible == 0) continue;
+                        on_device = on_device || !results[i].pixel_coordinates;
+                        if (!on_device) take<N>(results[i], out[i]);
+                    }
+                } catch (...) {
+                    (void) vmhip_batch_classify_end(batch_);
+                    throw;
+                }
+                classify_end();
+                if (on_device) return fetch<Model>();
+                const size_t classes = size_t(n_classes());
+                for (size_t i = 0; i < out.size(); ++i)
+                    if (results[i].classifications)
+                        out[i].classifications.assign(results[i].classifications, results[i].classifications + (size_t(results[i].n_visible) + 1) * classes);
+                return out;
             }
 
             /// Copy the frames' inputs to the device (images, poses, lenses, lookup ranges).
             template <template <typename> class Model>
             void stage(const std::vector<Frame<Model>>& frames) const {
-                stage_frames(frames, true, false);
+                stage_frames(frames, Stage::WAIT);
             }
             /// The same without waiting for the copies: they are queued ahead of the run and the call returns. The
             /// images must be page-locked (vmhip_host_alloc) and stay untouched until run() or wait() has returned.
             template <template <typename> class Model>
             void stage_async(const std::vector<Frame<Model>>& frames) const {
-                stage_frames(frames, false, false);
+                stage_frames(frames, Stage::ASYNC);
             }
 
         private:
+            /// How frames go to the device: waited for, not waited for, or as a call, which runs them and fills in `results` too.
+            enum class Stage { WAIT, ASYNC, CALL };
             template <template <typename> class Model>
-            void stage_frames(const std::vector<Frame<Model>>& frames, bool wait_for_copies, bool candidates) const {
+            void stage_frames(const std::vector<Frame<Model>>& frames, Stage how, std::vector<vmhip_result>* results = nullptr) const {
                 constexpr int N = Model<Scalar>::N_NEIGHBOURS;
+                const bool candidates = how == Stage::CALL;
                 staged_since_ = ++clock_;
                 staged_.assign(frames.size(), FrameData());
                 std::vector<vmhip_frame> flat(frames.size());
@@ -320,9 +346,11 @@ namespace engine {
                 staging_ = false;
                 vmhip_engine* e = handle(N);
                 if (!batch_) throw_on_error(vmhip_batch_create(e, &batch_));
-                if (!flat.empty())
-                    throw_on_error(wait_for_copies ? vmhip_batch_stage(batch_, flat.data(), int32_t(flat.size()), 1)
-                                                   : vmhip_batch_stage_async(batch_, flat.data(), int32_t(flat.size()), 1));
+                const int32_t n = int32_t(flat.size());
+                if (n > 0)
+                    throw_on_error(how == Stage::CALL   ? vmhip_batch_classify_begin(batch_, flat.data(), n, results->data())
+                                   : how == Stage::WAIT ? vmhip_batch_stage(batch_, flat.data(), n, 1)
+                                                        : vmhip_batch_stage_async(batch_, flat.data(), n, 1));
                 for (size_t i = 0; i < staged_.size(); ++i)
                     if (!staged_[i].untested.empty()) throw_on_error(vmhip_batch_set_untested(batch_, int32_t(i), staged_[i].untested.data(), int32_t(staged_[i].untested.size() / 2)));
             }
@@ -331,10 +359,6 @@ namespace engine {
             /// Run the staged frames on the device and wait; may be called repeatedly.
             void run() const {
                 if (batch_ && !staged_.empty()) throw_on_error(vmhip_batch_run(batch_));
-            }
-            /// The same ahead of fetch() and nothing else: the pass stores small results into the block that fetch() copies them from.
-            void run_held() const {
-                if (batch_ && !staged_.empty()) throw_on_error(vmhip_batch_run_held(batch_));
             }
             /// The same in two halves: the pass runs while the caller does something else (staging the next frames on
             /// a second engine, for one), and wait() blocks until it is done. fetch(), detect() and visible_counts()

@@ -328,7 +328,7 @@ __global__ __launch_bounds__(VMHIP_TILE) void vm_pack_geometry_kernel(VmBatchDev
     pack_tile_geometry(B, F, V, row0, dst + packed_geometry(B, f));
 }
 
-/* Last kernel of a pass.
+/* Last kernel of a pass, or of its two parts: a call of one frame has its verdict and its geometry before its image.
  *
  * Blocks [0, n_frames): what the host needs of the pass is written by the device straight into page-locked host memory
  * (block f: the head of frame f's ambiguity list; block 0 also the counts and the convolution kernel's count of waits that
@@ -346,19 +346,22 @@ __global__ __launch_bounds__(VMHIP_TILE) void vm_pack_geometry_kernel(VmBatchDev
  * the host, which sees the same counts, then fetches. */
 __global__ __launch_bounds__(VMHIP_TILE) void vm_publish_kernel(VmBatchDev B, VmPublish P) {
     if ((int) blockIdx.x < B.n_frames) {
-        const int f = blockIdx.x, n_counts = 2 * B.n_frames;
-        for (int t = threadIdx.x; t < P.amb_head; t += VMHIP_TILE) P.host_amb[(size_t) f * P.amb_head + t] = B.amb_list[(size_t) f * VMHIP_AMB_CAP + t];
-        if (f == 0) {
-            for (int t = threadIdx.x; t < n_counts; t += VMHIP_TILE) {
-                P.host_counts[t] = B.frame_V[t];
-                if (t >= B.n_frames) B.frame_V[t] = 0; /* the ambiguity counts lie behind the visible ones */
-            }
+        const int f = blockIdx.x;
+        if (P.verdict) {
+            for (int t = threadIdx.x; t < P.amb_head; t += VMHIP_TILE) P.host_amb[(size_t) f * P.amb_head + t] = B.amb_list[(size_t) f * VMHIP_AMB_CAP + t];
+            if (f == 0)
+                for (int t = threadIdx.x; t < 2 * B.n_frames; t += VMHIP_TILE) P.host_counts[t] = B.frame_V[t]; /* the ambiguity counts lie behind the visible ones */
+        }
+        if (P.ends && f == 0) {
+            __syncthreads();
+            for (int t = threadIdx.x; t < B.n_frames; t += VMHIP_TILE) B.amb_count[t] = 0;
             if (threadIdx.x == 0) {
                 *P.host_timeouts = P.timeouts ? *P.timeouts : 0u;
                 *B.epoch += 1;
                 *B.n_far_tiles = 0;
             }
         }
+        if (!P.verdict) return;
         __threadfence_system();
         __syncthreads();
         if (threadIdx.x == 0 && atomicAdd(B.published, 1u) + 1u == (uint32_t) B.n_frames) {
@@ -376,7 +379,7 @@ __global__ __launch_bounds__(VMHIP_TILE) void vm_publish_kernel(VmBatchDev B, Vm
     if (V == 0 || row0 > V) return;
     const VmDelivery to = *B.delivery;
     if (!to.block) return;
-    const size_t geometry = packed_geometry(B, B.n_frames), classes = P.classes ? packed_classes(B, B.n_frames, P.n_classes) : 0;
+    const size_t geometry = packed_geometry(B, B.n_frames), classes = P.n_classes ? packed_classes(B, B.n_frames, P.n_classes) : 0;
     if (geometry + classes > to.bytes) return;
     if (P.parts & VM_DELIVER_GEOMETRY) pack_tile_geometry(B, F, V, row0, to.block + packed_geometry(B, f));
     if (P.classes && (P.parts & VM_DELIVER_CLASSES)) {

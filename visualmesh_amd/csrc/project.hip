@@ -720,6 +720,84 @@ __device__ __forceinline__ float nbc_selu(float s) {
     const float alpha = 1.6732632423543772848170429916717f;
     return lambda * (s >= 0.0f ? s : __builtin_fmaf(alpha, __builtin_amdgcn_exp2f(s * 1.44269504088896340736f), -alpha));
 }
+/* The contraction, activation and store of a network's first layer for one row tile, by a block whose rows lie in LDS: the tile's 256 sampled rows, then
+ * its halo rows (staged_f), and the positions of every row's neighbours among them (nbl_rows). far_value(row of the tile, neighbour, channel) reads a
+ * neighbour that is not staged; a, bias4: the lane's weights and biases. */
+template <int NN, int CB, typename Far>
+__device__ __forceinline__ void first_layer_of_tile(const VmLayerDev& L, const float* staged_f, const uint16_t (*nbl_rows)[VMHIP_NBL_STRIDE], const float (&a)[NN + 1][CB],
+                                                    const nbc_v4f (&bias4)[CB], int n_rows, bool all_staged, size_t first_row, float* __restrict__ layer_out, Far far_value) {
+    constexpr int RBS = 4; /* row blocks of 16 per wave: a wave owns 64 rows of the tile */
+    constexpr int SLOTS = NN + 1;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q = lane >> 4, r16 = lane & 15;
+    const int c_out = L.c_out, activation = L.activation;
+    float x[RBS][SLOTS]; /* [row block][slot]: the lane's channel of the slot's source row */
+    /* block-uniform: every halo row of the tile has a slot (nearly always). The code is compiled for both cases,
+     * so that the usual one carries no test per position. */
+    auto gather = [&](auto checked_tag) {
+        constexpr bool CHECKED = decltype(checked_tag)::value;
+#pragma unroll
+        for (int rb = 0; rb < RBS; ++rb) {
+            const int row_t = min(wave * 64 + rb * 16 + r16, n_rows - 1); /* lanes past the tile's rows repeat its last row and store nothing */
+            const nbc_v4u positions = *reinterpret_cast<const nbc_v4u*>(nbl_rows[row_t]);
+            x[rb][0] = staged_f[row_t * 4 + q];
+#pragma unroll
+            for (int s = 0; s < NN; ++s) {
+                const uint32_t word = (s >> 1) == 0 ? positions.x : (s >> 1) == 1 ? positions.y : (s >> 1) == 2 ? positions.z : positions.w;
+                const uint32_t at = (s & 1) ? (word >> 16) : (word & 0xffffu);
+                /* a position that is not staged reads slot 0 here and is patched below */
+                x[rb][s + 1] = staged_f[(CHECKED && at == VMHIP_NBL_FAR ? 0u : at) * 4 + q];
+            }
+        }
+    };
+    if (all_staged) gather(std::false_type());
+    else gather(std::true_type());
+    if (!all_staged) { /* more halo rows than slots */
+#pragma unroll
+        for (int rb = 0; rb < RBS; ++rb) {
+            const int row_t = min(wave * 64 + rb * 16 + r16, n_rows - 1);
+#pragma unroll
+            for (int s = 0; s < NN; ++s) {
+                if (nbl_rows[row_t][s] == VMHIP_NBL_FAR) x[rb][s + 1] = far_value(row_t, s, q);
+            }
+        }
+    }
+    nbc_v4f acc[RBS][CB];
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+        for (int rb = 0; rb < RBS; ++rb) acc[rb][cb] = bias4[cb];
+#pragma unroll
+    for (int s = 0; s < SLOTS; ++s)
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+            for (int rb = 0; rb < RBS; ++rb) acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s][cb], x[rb][s], acc[rb][cb], 0, 0, 0);
+    /* one uniform branch for all the values */
+    auto for_each_value = [&](auto fn) {
+#pragma unroll
+        for (int rb = 0; rb < RBS; ++rb)
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[rb][cb][v] = fn(acc[rb][cb][v]);
+    };
+    if (activation == VMHIP_SELU) for_each_value([](float t) { return nbc_selu(t); });
+    else if (activation == VMHIP_RELU) for_each_value([](float t) { return fmaxf(t, 0.0f); });
+    else for_each_value([](float t) { return tanhf(t); });
+    /* the tile's output rows; a lane without a row, or a column block's padding, gets an offset the hardware drops */
+    const __amdgpu_buffer_rsrc_t out_rsrc =
+      __builtin_amdgcn_make_buffer_rsrc(layer_out + first_row * c_out, 0, VMHIP_TILE * c_out * 4, 0x00020000);
+#pragma unroll
+    for (int rb = 0; rb < RBS; ++rb) {
+        const int row_t = wave * 64 + rb * 16 + r16;
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) {
+            const int o = cb * 16 + q * 4;
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(nbc_v4u, acc[rb][cb]), out_rsrc,
+                                                   (row_t < n_rows && o < c_out) ? (uint32_t) (row_t * c_out + o) * 4u : 0xffffffffu, 0, 0);
+        }
+    }
+}
 template <bool WIDE, int NN, int CB>
 __global__ __launch_bounds__(VMHIP_TILE, CB == 1 ? (NN <= 6 ? 8 : 6) : CB == 2 ? 5 : 1) void vm_neighbourhood_kernel(VmBatchDev B, VmLayerDev L, const float* __restrict__ feat, float* __restrict__ layer_out) {
     static_assert(CB == 0 || (NN > 0 && NN <= VMHIP_NBL_STRIDE), "the fused first layer knows its neighbour count");
@@ -859,7 +937,6 @@ __global__ __launch_bounds__(VMHIP_TILE, CB == 1 ? (NN <= 6 ? 8 : 6) : CB == 2 ?
     }
 
     /* ---- first layer, part one: request what the contraction will read ---- */
-    constexpr int RBS = 4; /* row blocks of 16 per wave: a wave owns 64 rows of the tile */
     constexpr int SLOTS = NN + 1;
     float a[CB > 0 ? SLOTS : 1][CB > 0 ? CB : 1]; /* [slot][column block]: the lane's weight */
     nbc_v4u own_row = {0u, 0u, 0u, 0u}, halo_row = {0u, 0u, 0u, 0u};
@@ -958,86 +1035,73 @@ __global__ __launch_bounds__(VMHIP_TILE, CB == 1 ? (NN <= 6 ? 8 : 6) : CB == 2 ?
 
     /* ---- first layer, part two: contraction, activation, store ---- */
     if constexpr (CB > 0) {
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q = lane >> 4, r16 = lane & 15;
-        const int c_out = L.c_out, activation = L.activation;
         /* the rows the tile gathers, where the hash table was (every thread has passed the barrier after its last look at it) */
         nbc_v4u* const staged = reinterpret_cast<nbc_v4u*>(h_key);
         staged[threadIdx.x] = own_row;
         staged[VMHIP_TILE + threadIdx.x] = halo_row;
         __syncthreads();
-        const float* const staged_f = reinterpret_cast<const float*>(h_key);
-        float x[RBS][SLOTS]; /* [row block][slot]: the lane's channel of the slot's source row */
-        /* block-uniform: every halo row of the tile has a slot (nearly always). The code is compiled for both cases,
-         * so that the usual one carries no test per position. */
-        const bool all_staged = total <= cap;
-        auto gather = [&](auto checked_tag) {
-            constexpr bool CHECKED = decltype(checked_tag)::value;
-#pragma unroll
-            for (int rb = 0; rb < RBS; ++rb) {
-                const int row_t = min(wave * 64 + rb * 16 + r16, n_rows - 1); /* lanes past the tile's rows repeat its last row and store nothing */
-                const nbc_v4u positions = *reinterpret_cast<const nbc_v4u*>(nbl_rows[row_t]);
-                x[rb][0] = staged_f[row_t * 4 + q];
-#pragma unroll
-                for (int s = 0; s < NN; ++s) {
-                    const uint32_t word = (s >> 1) == 0 ? positions.x : (s >> 1) == 1 ? positions.y : (s >> 1) == 2 ? positions.z : positions.w;
-                    const uint32_t at = (s & 1) ? (word >> 16) : (word & 0xffffu);
-                    /* a position that is not staged reads slot 0 here and is patched below */
-                    x[rb][s + 1] = staged_f[(CHECKED && at == VMHIP_NBL_FAR ? 0u : at) * 4 + q];
-                }
-            }
-        };
-        if (all_staged) gather(std::false_type());
-        else gather(std::true_type());
-        if (!all_staged) { /* more halo rows than slots: those rows' numbers from the table this block has just written */
-#pragma unroll
-            for (int rb = 0; rb < RBS; ++rb) {
-                const int row_t = min(wave * 64 + rb * 16 + r16, n_rows - 1);
-#pragma unroll
-                for (int s = 0; s < NN; ++s) {
-                    if (nbl_rows[row_t][s] == VMHIP_NBL_FAR) {
-                        const int g = read_element(nb_out, (Off) (row0 + row_t) * nb_stride + (Off) s);
-                        x[rb][s + 1] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(sampled_rows(), g * 16 + q * 4, 0, 0));
-                    }
-                }
-            }
-        }
-        nbc_v4f acc[RBS][CB];
-#pragma unroll
-        for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-            for (int rb = 0; rb < RBS; ++rb) acc[rb][cb] = bias4[cb];
-#pragma unroll
-        for (int s = 0; s < SLOTS; ++s)
-#pragma unroll
-            for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-                for (int rb = 0; rb < RBS; ++rb) acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s][cb], x[rb][s], acc[rb][cb], 0, 0, 0);
-        /* one uniform branch for all the values */
-        auto for_each_value = [&](auto fn) {
-#pragma unroll
-            for (int rb = 0; rb < RBS; ++rb)
-#pragma unroll
-                for (int cb = 0; cb < CB; ++cb)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) acc[rb][cb][v] = fn(acc[rb][cb][v]);
-        };
-        if (activation == VMHIP_SELU) for_each_value([](float t) { return nbc_selu(t); });
-        else if (activation == VMHIP_RELU) for_each_value([](float t) { return fmaxf(t, 0.0f); });
-        else for_each_value([](float t) { return tanhf(t); });
-        /* the tile's output rows; a lane without a row, or a column block's padding, gets an offset the hardware drops */
-        const __amdgpu_buffer_rsrc_t out_rsrc =
-          __builtin_amdgcn_make_buffer_rsrc(layer_out + ((size_t) row_base + row0) * c_out, 0, VMHIP_TILE * c_out * 4, 0x00020000);
-#pragma unroll
-        for (int rb = 0; rb < RBS; ++rb) {
-            const int row_t = wave * 64 + rb * 16 + r16;
-#pragma unroll
-            for (int cb = 0; cb < CB; ++cb) {
-                const int o = cb * 16 + q * 4;
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(nbc_v4u, acc[rb][cb]), out_rsrc,
-                                                       (row_t < n_rows && o < c_out) ? (uint32_t) (row_t * c_out + o) * 4u : 0xffffffffu, 0, 0);
-            }
-        }
+        first_layer_of_tile<NN, CB>(L, reinterpret_cast<const float*>(h_key), nbl_rows, a, bias4, n_rows, total <= cap, (size_t) row_base + row0, layer_out, [&](int row_t, int slot, int q) {
+            const int g = read_element(nb_out, (Off) (row0 + row_t) * nb_stride + (Off) slot); /* from the table this block has just written */
+            return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(sampled_rows(), g * 16 + q * 4, 0, 0));
+        });
     }
+}
+
+/* The sampled rows of a pass whose geometry was there before its images (a call of one frame): one thread per row, what vm_compact_kernel does for a candidate. */
+__device__ __forceinline__ float4 sampled_row(const VmBatchDev& B, const VmFrame& F, int V, int row) {
+    if (row >= V) return make_float4(-1.0f, -1.0f, -1.0f, -1.0f); /* the off-screen row, engine/cpu/engine.hpp:205-206 */
+    return sample_image(F, B.row_px[(size_t) F.row_base + row]);
+}
+__global__ __launch_bounds__(VMHIP_TILE) void vm_sample_kernel(VmBatchDev B, float4* __restrict__ feat) {
+    const int tile = blockIdx.x;
+    if (tile >= vm_row_tiles(B)) return;
+    const int f = B.row_tile_frame[tile];
+    const VmFrame& F = B.frames[f];
+    const int V = B.frame_V[f], row = (tile - F.row_tile0) * VMHIP_TILE + threadIdx.x;
+    if (row <= V) feat[(size_t) F.row_base + row] = sampled_row(B, F, V, row);
+}
+
+/* The same with the network's first layer: the block samples its tile's rows and its halo rows, 0.4 times as many again, into LDS and goes on as vm_neighbourhood_kernel
+ * does, with the same bits. One launch and no 16-byte rows in memory in between. Bound by latency at a frame's 256 to 500 tiles: descriptor, halo numbers, pixels,
+ * texels, one after the other. 10.7 us for 65 000 rows of an RGBA image (16
+ * channels out), 17.4 for 128 000 of a Bayer one (24, eight neighbours); inside the compaction and the neighbourhoods the same work takes 5 and 9 us less, which a call
+ * gets back several times over: see batch_launch_call in api.hip. */
+template <int NN, int CB>
+__global__ __launch_bounds__(VMHIP_TILE) void vm_sample_conv_kernel(VmBatchDev B, VmLayerDev L, float* __restrict__ layer_out) {
+    __shared__ __align__(16) float4 staged[VMHIP_TILE + VMHIP_HALO_MAX];
+    __shared__ __align__(16) uint16_t nbl_rows[VMHIP_TILE][VMHIP_NBL_STRIDE];
+    const int tile = blockIdx.x;
+    if (tile >= vm_row_tiles(B)) return;
+    const int f = B.row_tile_frame[tile];
+    const VmFrame& F = B.frames[f];
+    const int V = B.frame_V[f], row_base = F.row_base, row0 = (tile - F.row_tile0) * VMHIP_TILE;
+    const int4 desc = B.tile_desc[tile]; /* {first row, rows in use, halo rows, frame's first row} */
+    const int n_rows = desc.y;
+    if (n_rows <= 0) return;
+    const int row_t = min((int) threadIdx.x, n_rows - 1); /* threads past the tile's rows redo its last row */
+    const bool has_halo = (int) threadIdx.x < desc.z;
+    const int halo = has_halo ? (int) B.tile_halo[(size_t) tile * VMHIP_HALO_MAX + threadIdx.x] - row_base : 0;
+    *reinterpret_cast<nbc_v4u*>(nbl_rows[threadIdx.x]) = *reinterpret_cast<const nbc_v4u*>(B.row_nbl + ((size_t) row_base + row0 + row_t) * VMHIP_NBL_STRIDE);
+    float a[NN + 1][CB];
+    nbc_v4f bias4[CB];
+    const VM_GLOBAL float* const w = in_device_memory(reinterpret_cast<const float*>(L.w_mfma));
+#pragma unroll
+    for (int s = 0; s <= NN; ++s)
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) a[s][cb] = w[(s * CB + cb) * 64 + (threadIdx.x & 63)];
+    const int q4 = ((threadIdx.x & 63) >> 4) * 4;
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) {
+        bias4[cb] = nbc_v4f{0.0f, 0.0f, 0.0f, 0.0f};
+        if (cb * 16 + q4 < L.c_out) bias4[cb] = *reinterpret_cast<const VM_GLOBAL nbc_v4f*>(in_device_memory(L.b) + cb * 16 + q4); /* c_out is a multiple of 4 */
+    }
+    staged[threadIdx.x] = sampled_row(B, F, V, row0 + row_t);
+    if (has_halo) staged[VMHIP_TILE + threadIdx.x] = sampled_row(B, F, V, halo);
+    __syncthreads();
+    first_layer_of_tile<NN, CB>(L, reinterpret_cast<const float*>(staged), nbl_rows, a, bias4, n_rows, desc.z < B.halo_cap, (size_t) row_base + row0, layer_out, [&](int r, int slot, int q) {
+        const float4 v = sampled_row(B, F, V, B.row_nb[((size_t) row_base + row0 + r) * B.nb_stride + slot]);
+        return q == 0 ? v.x : q == 1 ? v.y : q == 2 ? v.z : v.w;
+    });
 }
 
 }  // namespace
@@ -1116,6 +1180,30 @@ int vm_launch_neighbourhood_conv(const VmBatchDev& B, const VmLayerDev& L, const
     case NN:                                                                              \
         if (B.wide_offsets) launch_neighbourhood_conv<true, NN>(B, L, in, out, stream);   \
         else launch_neighbourhood_conv<false, NN>(B, L, in, out, stream);                 \
+        break;
+    switch (B.uniform_nn) {
+        X(4)
+        X(6)
+        X(8)
+        default: return -1;
+    }
+#undef X
+    return 0;
+}
+void vm_launch_sample(const VmBatchDev& B, float* feat, hipStream_t stream) {
+    if (B.n_row_tiles > 0) hipLaunchKernelGGL(vm_sample_kernel, dim3(B.n_row_tiles), dim3(VMHIP_TILE), 0, stream, B, reinterpret_cast<float4*>(feat));
+}
+int vm_launch_sample_conv(const VmBatchDev& B, const VmLayerDev& L, float* out, hipStream_t stream, const char** kernel_name) {
+    if (!vm_neighbourhood_conv_supported(L.c_in, L.c_out, L.slots, L.activation) || !B.row_nbl || !L.w_mfma || !L.b || L.in_bf16 || L.out_bf16 || L.arith_bf16
+        || B.uniform_nn != L.slots - 1)
+        return -1;
+    if (kernel_name) *kernel_name = vm_kernel_name("sample_conv", L.c_in, L.c_out, L.slots);
+    if (B.n_row_tiles <= 0) return 0;
+    const dim3 grid(B.n_row_tiles), block(VMHIP_TILE);
+#define X(NN)                                                                                                            \
+    case NN:                                                                                                             \
+        if (L.c_out <= 16) hipLaunchKernelGGL((vm_sample_conv_kernel<NN, 1>), grid, block, 0, stream, B, L, out);        \
+        else hipLaunchKernelGGL((vm_sample_conv_kernel<NN, 2>), grid, block, 0, stream, B, L, out);                      \
         break;
     switch (B.uniform_nn) {
         X(4)

@@ -258,15 +258,16 @@ void vm_launch_stream_probe(const void* src, void* dst, size_t rows, int read_by
  * stored by the device into page-locked host memory (device-visible pointers); `parts` of the results into the block of B.delivery. */
 enum { VM_DELIVER_GEOMETRY = 1, VM_DELIVER_CLASSES = 2 };
 struct VmPublish {
+    int32_t verdict, ends;    /* the host hears of counts and ambiguities; the pass is over (timeouts, and everything left as the next pass expects it) */
     int32_t amb_head;
     int32_t parts;            /* VM_DELIVER_*: at most VM_GEOMETRY_FRAMES frames, staged with their tile tables */
     const unsigned int* timeouts;
     int32_t* host_counts;
     int2* host_amb;
     uint32_t* host_timeouts;
-    uint32_t* host_serial;    /* gets VmDelivery::serial when everything above is there */
-    const float* classes;     /* [rows][n_classes], or null */
-    int32_t n_classes;
+    uint32_t* host_serial;    /* with the verdict: gets VmDelivery::serial when everything above is there */
+    const float* classes;     /* [rows][n_classes]; null while there are none */
+    int32_t n_classes;        /* 0: the results have no classifications */
     uint8_t* classes_packed;  /* device memory with room for all classifications, to leave them there; null: into the block */
 };
 void vm_launch_publish(const VmBatchDev& B, const VmPublish& P, hipStream_t stream);
@@ -278,6 +279,10 @@ void vm_launch_neighbourhood(const VmBatchDev& B, hipStream_t stream); /* also t
  * (then nothing was launched) */
 bool vm_neighbourhood_conv_supported(int c_in, int c_out, int slots, int activation);
 int vm_launch_neighbourhood_conv(const VmBatchDev& B, const VmLayerDev& L, const float* in, float* out, hipStream_t stream, const char** kernel_name);
+/* sampling as launches of their own, behind a vm_launch_compact and a vm_launch_neighbourhood without it: the sampled rows, or what
+ * vm_launch_neighbourhood_conv makes of them (a negative value as there) */
+void vm_launch_sample(const VmBatchDev& B, float* feat, hipStream_t stream);
+int vm_launch_sample_conv(const VmBatchDev& B, const VmLayerDev& L, float* out, hipStream_t stream, const char** kernel_name);
 /* in -> out over the row space; returns 0 or a negative status if the shape is unsupported */
 int vm_launch_conv(const VmBatchDev& B, const VmLayerDev& L, const float* in, float* out, hipStream_t stream,
                    const char** kernel_name);

@@ -138,17 +138,22 @@ class Engine:
         n_out, nn = self.network.n_out, m.n_neighbours
         img = np.ascontiguousarray(image)
         r = native.Result()
-        native.host_check(self._lib.vmh_engine_classify_held(self.ptr, m.ptr, _fp(H), C.byref(lens), img.ctypes.data, fcc, C.byref(r)))
-        V = r.n_visible
+        native.host_check(self._lib.vmh_engine_classify_begin(self.ptr, m.ptr, _fp(H), C.byref(lens), img.ctypes.data, fcc, C.byref(r)))
+        V, held = r.n_visible, bool(r.pixel_coordinates)
+        try:  # the network is still at work
+            if held:
+                px, nb, gidx = (self._taken(r.pixel_coordinates, (V, 2), np.float32), self._taken(r.neighbourhood, (V + 1, nn), np.int32),
+                                self._taken(r.global_indices, (V,), np.int32))
+        finally:
+            native.host_check(self._lib.vmh_engine_classify_end(self.ptr))
         if V == 0:
             return dict(px=np.zeros((0, 2), np.float32), nb=np.zeros((0, nn), np.int32), gidx=np.zeros(0, np.int32), cls=np.zeros((0, n_out), np.float32))
-        if not r.pixel_coordinates:  # more than the engine holds: straight from the device
+        if not held:  # more than the engine holds: straight from the device
             px, nb, gidx, cls = np.empty((V, 2), np.float32), np.empty((V + 1, nn), np.int32), np.empty(V, np.int32), np.empty((V + 1, n_out), np.float32)
             r = native.Result(V, 0, _fp(px), _ip(gidx), _ip(nb), _fp(cls))
             native.hip_check(native.hip().vmhip_batch_fetch(self.native_batch(), C.byref(r)))
             return dict(px=px, nb=nb, gidx=gidx, cls=cls)
-        return dict(px=self._taken(r.pixel_coordinates, (V, 2), np.float32), nb=self._taken(r.neighbourhood, (V + 1, nn), np.int32),
-                    gidx=self._taken(r.global_indices, (V,), np.int32), cls=self._taken(r.classifications, (V + 1, n_out), np.float32))
+        return dict(px=px, nb=nb, gidx=gidx, cls=self._taken(r.classifications, (V + 1, n_out), np.float32))
 
     def __call__(self, mesh, Hoc, lens, image=None, fcc=None):
         if image is None:
