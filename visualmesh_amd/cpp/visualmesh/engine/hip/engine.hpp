@@ -303,12 +303,14 @@ namespace engine {
             }
 
         private:
-            /// How frames go to the device: waited for, not waited for, or as a call, which runs them and fills in `results` too.
-            enum class Stage { WAIT, ASYNC, CALL };
+            /// How frames go to the device: waited for, not waited for, as a call, which runs them and fills in `results` too, or as a batch of a stream of
+            /// batches, which starts them and fills in `visible`.
+            enum class Stage { WAIT, ASYNC, CALL, STREAM };
             template <template <typename> class Model>
-            void stage_frames(const std::vector<Frame<Model>>& frames, Stage how, std::vector<vmhip_result>* results = nullptr) const {
+            void stage_frames(const std::vector<Frame<Model>>& frames, Stage how, std::vector<vmhip_result>* results = nullptr, const Engine* first = nullptr,
+                              std::vector<int32_t>* visible = nullptr) const {
                 constexpr int N = Model<Scalar>::N_NEIGHBOURS;
-                const bool candidates = how == Stage::CALL;
+                const bool candidates = how == Stage::CALL || how == Stage::STREAM;
                 staged_since_ = ++clock_;
                 staged_.assign(frames.size(), FrameData());
                 std::vector<vmhip_frame> flat(frames.size());
@@ -348,7 +350,8 @@ namespace engine {
                 if (!batch_) throw_on_error(vmhip_batch_create(e, &batch_));
                 const int32_t n = int32_t(flat.size());
                 if (n > 0)
-                    throw_on_error(how == Stage::CALL   ? vmhip_batch_classify_begin(batch_, flat.data(), n, results->data())
+                    throw_on_error(how == Stage::CALL     ? vmhip_batch_classify_begin(batch_, flat.data(), n, results->data())
+                                   : how == Stage::STREAM ? vmhip_batch_stream_begin(batch_, first->batch_, flat.data(), n, visible->data())
                                    : how == Stage::WAIT ? vmhip_batch_stage(batch_, flat.data(), n, 1)
                                                         : vmhip_batch_stage_async(batch_, flat.data(), n, 1));
                 for (size_t i = 0; i < staged_.size(); ++i)
@@ -418,6 +421,22 @@ namespace engine {
                 if (results.size() != staged_.size()) throw std::invalid_argument("fetch_into_async: one result per staged frame");
                 if (!results.empty()) throw_on_error(vmhip_batch_fetch_async(batch_, results.data()));
             }
+            /// One batch of a stream of batches, by engines that take turns, step by step (see vmhip_batch_stream_begin; Pipeline takes them). `first` is the
+            /// same engine for all that take turns, has streamed a batch before the others do, and outlives them.
+            template <template <typename> class Model>
+            std::vector<int32_t> stream_begin(const std::vector<Frame<Model>>& frames, const Engine& first) const {
+                std::vector<int32_t> visible(frames.size());
+                stage_frames(frames, Stage::STREAM, nullptr, &first, &visible);
+                return visible;
+            }
+            void stream_layers() const { throw_on_error(vmhip_batch_stream_layers(batch_)); }
+            void stream_geometry(void* block, size_t bytes, std::vector<vmhip_result>& results) const {
+                results.assign(staged_.size(), vmhip_result{});
+                throw_on_error(vmhip_batch_stream_geometry(batch_, block, bytes, results.data()));
+            }
+            void stream_classes() const { throw_on_error(vmhip_batch_stream_classes(batch_)); }
+            void stream_images() const { throw_on_error(vmhip_batch_stream_images(batch_)); }
+            void stream_end() const { throw_on_error(vmhip_batch_stream_end(batch_)); }
             void fetch_wait() const {
                 if (batch_ && !staged_.empty()) throw_on_error(vmhip_batch_fetch_wait(batch_));
             }
@@ -1026,10 +1045,9 @@ namespace engine {
         };
 
         /**
-         * Three engines taking turns, so that the upload of one batch, the kernels of the one before and the download of
-         * the one before that run at the same time: what a caller otherwise writes by hand with stage_async / run_async /
-         * wait / fetch_into_async / fetch_wait on three Engine objects. No counterpart in the reference, whose benchmark
-         * runs one frame at a time per engine (example/benchmark.cpp:50-58).
+         * Three engines taking turns, so that the uploads of one batch after the other leave no gap on the bus, with the geometry of a batch
+         * worked out and on its way home while its images come, and its layers behind them (Engine::stream_begin). No counterpart in the
+         * reference, whose benchmark runs one frame at a time per engine (example/benchmark.cpp:50-58).
          *
          *     Pipeline<float> pipe(network);
          *     for (;;) { if (auto* done = pipe.submit(next_frames())) consume(*done); }   // results of the batch two submits ago
@@ -1050,8 +1068,7 @@ namespace engine {
             ~Pipeline() {
                 for (Slot& s : slots_) {
                     try {
-                        if (s.running) s.engine->wait();
-                        if (s.fetching) s.engine->fetch_wait();
+                        if (s.busy) s.end();
                     } catch (...) {
                     }
                     if (s.block) vmhip_host_free(s.block);
@@ -1065,17 +1082,33 @@ namespace engine {
             template <template <typename> class Model>
             const std::vector<vmhip_result>* submit(const std::vector<typename Engine<Scalar>::template Frame<Model>>& frames) {
                 Slot& now = slots_[step_ % 3];
-                now.engine->stage_async(frames);
-                now.engine->run_async();
-                now.running = true;
-                now.neighbours = Model<Scalar>::N_NEIGHBOURS;
+                Slot& oldest = slots_[(step_ + 1) % 3];
+                if (now.busy) now.end();  // an earlier call failed before it had waited for these
+                now.results.clear();
+                now.submitted = true;
+                if (!frames.empty()) {
+                    now.engine->stream_begin(frames, *slots_[0].engine);
+                    now.busy = true, now.copied = false;
+                    const size_t need = std::max<size_t>(now.engine->packed_size(), 256);
+                    if (need > now.block_bytes) {
+                        if (now.block) vmhip_host_free(now.block);
+                        now.block = vmhip_host_alloc(need + need / 8);
+                        now.block_bytes = now.block ? need + need / 8 : 0;
+                        if (!now.block) throw std::system_error(VMHIP_ERR_HIP, hip_error_category(), "Pipeline: no page-locked memory for the results");
+                    }
+                    oldest.classes();  // ahead of the next copy in that direction
+                    now.engine->stream_geometry(now.block, now.block_bytes, now.results);
+                    Slot& previous = slots_[(step_ + 2) % 3];
+                    if (previous.busy) previous.engine->stream_images();  // one upload at a time
+                    now.engine->stream_layers();
+                }
                 return advance();
             }
             /// Drain: the results of the batches still in flight, oldest first, then nullptr.
             const std::vector<vmhip_result>* flush() {
                 for (int turn = 0; turn < 2; ++turn) {
                     bool in_flight = false;
-                    for (const Slot& s : slots_) in_flight = in_flight || s.running || s.fetching;
+                    for (const Slot& s : slots_) in_flight = in_flight || s.submitted;
                     if (!in_flight) return nullptr;
                     if (const std::vector<vmhip_result>* done = advance()) return done;
                 }
@@ -1096,56 +1129,31 @@ namespace engine {
         private:
             struct Slot {
                 std::unique_ptr<Engine<Scalar>> engine;
-                bool running = false, fetching = false;
-                int neighbours = 0;
+                bool submitted = false, busy = false, copied = false;  ///< results to be returned; an engine at work for them; their last copy queued
                 void* block = nullptr;
                 size_t block_bytes = 0;
                 std::vector<vmhip_result> results;
+                void classes() {
+                    if (busy && !copied) engine->stream_classes();
+                    copied = true;
+                }
+                void end() {
+                    const bool wait = busy;
+                    if (wait) classes();
+                    busy = false;
+                    if (wait) engine->stream_end();
+                }
             };
-            static size_t pad(size_t n) { return (n + 255) / 256 * 256; }
-
             const std::vector<vmhip_result>* advance() {
-                Slot& previous = slots_[(step_ + 2) % 3];  // submitted one call ago: its kernels finish, its download starts
-                Slot& oldest = slots_[(step_ + 1) % 3];    // submitted two calls ago: its download finishes
+                Slot& previous = slots_[(step_ + 2) % 3];  // submitted one call ago: its images are to be read when this call returns
+                Slot& oldest = slots_[(step_ + 1) % 3];    // submitted two calls ago: to be finished
                 ++step_;
-                /* The oldest batch's download is finished before the next one is queued: with the tail of one download and
-                 * the head of the next in flight together, the upload that runs beside them takes longer (2.0-2.1 ms per
-                 * batch instead of 1.8 on the benchmark's batches). */
                 const std::vector<vmhip_result>* done = nullptr;
-                if (previous.running) previous.engine->wait();
-                if (oldest.fetching) {
-                    oldest.engine->fetch_wait();
-                    oldest.fetching = false;
-                    done = &oldest.results;
-                }
-                if (previous.running) {
-                    previous.running = false;
-                    const std::vector<int32_t> visible = previous.engine->visible_counts();
-                    const size_t classes = size_t(previous.engine->n_classes()), nn = size_t(previous.neighbours);
-                    size_t need = 0;
-                    for (int32_t v : visible)
-                        if (v > 0) need += pad(8 * size_t(v)) + pad(4 * size_t(v)) + pad(4 * (size_t(v) + 1) * nn) + pad(4 * (size_t(v) + 1) * classes);
-                    if (need > previous.block_bytes) {
-                        if (previous.block) vmhip_host_free(previous.block);
-                        previous.block = vmhip_host_alloc(need + need / 8);
-                        previous.block_bytes = previous.block ? need + need / 8 : 0;
-                        if (!previous.block) throw std::system_error(VMHIP_ERR_HIP, hip_error_category(), "Pipeline: no page-locked memory for the results");
-                    }
-                    previous.results.assign(visible.size(), vmhip_result{});
-                    char* at = static_cast<char*>(previous.block);
-                    for (size_t i = 0; i < visible.size(); ++i) {
-                        const size_t v = size_t(visible[i]);
-                        vmhip_result& r = previous.results[i];
-                        r.capacity = int32_t(v);
-                        if (v == 0) continue;
-                        r.pixel_coordinates = reinterpret_cast<float*>(at), at += pad(8 * v);
-                        r.global_indices = reinterpret_cast<int32_t*>(at), at += pad(4 * v);
-                        r.neighbourhood = reinterpret_cast<int32_t*>(at), at += pad(4 * (v + 1) * nn);
-                        r.classifications = reinterpret_cast<float*>(at), at += pad(4 * (v + 1) * classes);
-                    }
-                    previous.engine->fetch_into_async(previous.results);
-                    previous.fetching = true;
-                }
+                const bool finish = oldest.submitted;
+                oldest.submitted = false;
+                if (finish) done = &oldest.results;
+                if (previous.busy) previous.engine->stream_images();
+                if (oldest.busy) oldest.end();
                 return done;
             }
 

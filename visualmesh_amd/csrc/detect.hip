@@ -377,13 +377,16 @@ __global__ __launch_bounds__(VMHIP_TILE) void vm_publish_kernel(VmBatchDev B, Vm
     const VmFrame& F = B.frames[f];
     const int V = B.frame_V[f], row0 = (tile - F.row_tile0) * VMHIP_TILE;
     if (V == 0 || row0 > V) return;
-    const VmDelivery to = *B.delivery;
-    if (!to.block) return;
-    const size_t geometry = packed_geometry(B, B.n_frames), classes = P.n_classes ? packed_classes(B, B.n_frames, P.n_classes) : 0;
-    if (geometry + classes > to.bytes) return;
-    if (P.parts & VM_DELIVER_GEOMETRY) pack_tile_geometry(B, F, V, row0, to.block + packed_geometry(B, f));
+    uint8_t* base = P.classes_packed;
+    if (!base || (P.parts & VM_DELIVER_GEOMETRY)) {
+        const VmDelivery to = *B.delivery;
+        if (!to.block) return;
+        const size_t geometry = packed_geometry(B, B.n_frames), classes = P.n_classes ? packed_classes(B, B.n_frames, P.n_classes) : 0;
+        if (geometry + classes > to.bytes) return;
+        if (!base) base = to.block + geometry;
+        if (P.parts & VM_DELIVER_GEOMETRY) pack_tile_geometry(B, F, V, row0, to.block + packed_geometry(B, f));
+    }
     if (P.classes && (P.parts & VM_DELIVER_CLASSES)) {
-        uint8_t* const base = P.classes_packed ? P.classes_packed : to.block + geometry;
         const size_t row_bytes = 4 * (size_t) P.n_classes;
         pack_piece(P.classes + ((size_t) F.row_base + row0) * P.n_classes, base + packed_classes(B, f, P.n_classes) + row_bytes * row0,
                    row_bytes * (size_t) min(VMHIP_TILE, V + 1 - row0));
