@@ -45,3 +45,27 @@ def test_the_same_bytes_as_array_by_array(ks, classes, model, blind):
         _same([engine(f["mesh"], f["Hoc"], f["lens"], f["image"], f["fourcc"])], [w])
         if len(w["gidx"]):
             _same([engine.project(f["mesh"], f["Hoc"], f["lens"])], [{key: w[key] for key in ("px", "nb", "gidx")}])
+
+
+@pytest.mark.parametrize("precision", [native.FP32, native.BF16, native.SPLIT], ids=["fp32", "bf16", "split"])
+@pytest.mark.parametrize("frames,blind,halo_cap", [(10, (), None), (10, (0, 4, 5, 9), None), (12, (1,), 20), (1, (), None)], ids=["four groups", "blind frames", "far neighbours", "one frame"])
+def test_the_last_two_layers_by_groups_of_frames(precision, frames, blind, halo_cap, monkeypatch):
+    """More than 8 MB of classifications behind 64-wide layers: the same bits as with all frames at once, which the first passes and every other fetch have."""
+    if halo_cap is not None:
+        monkeypatch.setenv("VMHIP_HALO_CAP", str(halo_cap))
+    rng = np.random.default_rng(7)
+    lens, sky = native.make_lens(1280, 1024, wl.EQUISOLID, 420.0, math.pi), native.make_lens(1280, 1024, wl.RECTILINEAR, 700.0, math.pi / 2)
+    mesh, image = eng.Mesh(wl.RING6, wl.SPHERE, 0.0949, 1.2, 24.5 if frames == 1 else 7.6, 20.0), wl.random_image(rng, 1280, 1024, 4)
+    batch = [dict(mesh=mesh, Hoc=wl.make_hoc(1.2, math.radians(-80.0 if i in blind else rng.uniform(20, 50)), 0.0, rng.uniform(-3, 3)), lens=sky if i in blind else lens, image=image,
+                  fourcc=wl.fourcc("RGBA")) for i in range(frames)]
+    engine = eng.Engine(wl.glorot_network(np.random.default_rng(3), [3, 64, 64, 64, 4], 6, wl.SELU), wl.RING6, precision)
+    engine.stage(batch)
+    assert sum(16 * int((r[:, 1] - r[:, 0]).sum()) for r in (engine.staged_ranges(i) for i in range(frames))) > 8 << 20
+    want = None
+    for turn in range(5):
+        engine.run()
+        got = engine.fetch_packed()
+        if want is None:
+            want = [{key: a.copy() for key, a in g.items()} for g in got]
+        _same(got, want)
+    _same(engine.fetch_pinned(), want)

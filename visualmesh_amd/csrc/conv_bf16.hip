@@ -227,11 +227,11 @@ __global__ __launch_bounds__(256) void vm_conv_bf16_kernel(VmBatchDev B, VmLayer
     float* const xch = b_lds + CH;
 
     /* half tiles in use, and this block's share: XCD-aware (block b works for XCD b % 8 on a contiguous eighth) */
-    const int n_tiles = B.active_h[B.n_frames];
+    const int n_tiles = B.active_h[L.frame_end], t_first = B.active_h[L.frame_begin]; /* of the launch's frames: half tiles t_first to n_tiles */
     const int xcd = blockIdx.x & 7, lb = blockIdx.x >> 3, gx = gridDim.x >> 3;
-    const int per_xcd = (n_tiles + 7) >> 3;
-    const int t_end = min(n_tiles, (xcd + 1) * per_xcd);
-    const int tile0 = xcd * per_xcd + lb;
+    const int per_xcd = (n_tiles - t_first + 7) >> 3;
+    const int t_end = min(n_tiles, t_first + (xcd + 1) * per_xcd);
+    const int tile0 = t_first + xcd * per_xcd + lb;
     if (tile0 >= t_end) return; /* the whole block leaves before any barrier or LDS load */
     const int count = (t_end - tile0 + gx - 1) / gx; /* half tiles of this block: tile0 + k * gx, k < count */
 

@@ -88,11 +88,11 @@ __global__ __launch_bounds__(256) void vm_conv_x3_kernel(VmBatchDev B, VmLayerDe
     v4u* const low_lds = reinterpret_cast<v4u*>(b_lds + C) + cb * (LOW_SLOTS * STAGES * 2 * 64) + lane;
 
     /* half tiles in use, and this block's share: XCD-aware (block b works for XCD b % 8 on a contiguous eighth) */
-    const int n_tiles = B.active_h[B.n_frames];
+    const int n_tiles = B.active_h[L.frame_end], t_first = B.active_h[L.frame_begin]; /* of the launch's frames: half tiles t_first to n_tiles */
     const int xcd = blockIdx.x & 7, lb = blockIdx.x >> 3, gx = gridDim.x >> 3;
-    const int per_xcd = (n_tiles + 7) >> 3;
-    const int t_end = min(n_tiles, (xcd + 1) * per_xcd);
-    const int tile0 = xcd * per_xcd + lb;
+    const int per_xcd = (n_tiles - t_first + 7) >> 3;
+    const int t_end = min(n_tiles, t_first + (xcd + 1) * per_xcd);
+    const int tile0 = t_first + xcd * per_xcd + lb;
     const int count = tile0 < t_end ? (t_end - tile0 + gx - 1) / gx : 0; /* half tiles of this block: tile0 + k * gx, k < count */
 
     /* the wave's weights: [cb][stage][slot][step][h, m, l][lane] 16 bytes each */
@@ -380,7 +380,9 @@ __global__ __launch_bounds__(256) void vm_conv_x3_kernel(VmBatchDev B, VmLayerDe
     constexpr int DEEP = 6, PER_TILE = CBW;
     const int n_far = B.active_h[B.n_frames + 1] * PER_TILE;
     for (int t = blockIdx.x; t < n_far; t += gridDim.x) {
-        const uint32_t* const note = B.tile_note_h + (size_t) B.far_h[t / PER_TILE] * NOTE;
+        const int number = B.far_h[t / PER_TILE];
+        if (number < t_first || number >= n_tiles) continue; /* another launch's: the rows that it reads may no longer be what they were */
+        const uint32_t* const note = B.tile_note_h + (size_t) number * NOTE;
         const uint32_t first = note[0], in_use = note[1], frame_row = note[3];
         const uint32_t row = (uint32_t) (((t % PER_TILE) * (4 / CBW) + rw) * 32 + r32), own = min(row, in_use - 1);
         uint32_t from[SLOTS];

@@ -203,6 +203,7 @@ struct VmLayerDev {
     int32_t arith_bf16; /* bf16 products with fp32 accumulation (weights in w_mfma are bf16 then) */
     const float* w_flow; /* the fp32 w_mfma weights in the order conv_flow.hip keeps them in LDS, or null */
     const void* w_x3;    /* three bf16 parts of every weight in conv_x3.hip's order, or null */
+    int32_t frame_begin, frame_end; /* the frames that conv_bf16.hip, conv_x3.hip and the sliced kernel of conv_narrow.hip work on; the others take all */
 };
 
 /* Device side of the detection step (detect.hip): every array is indexed like the row space, a frame's entries
@@ -358,6 +359,7 @@ hipError_t vm_flow_set_poll_limit(int polls); /* process wide; tests of the give
 /* layers with at most four output channels on v_mfma_f32_4x4x1 (64 rows x 4 channels per instruction), staged like
  * conv_flow.hip (conv_narrow.hip); reads the plain row-major weights */
 bool vm_narrow_supported(int c_in, int c_out, int slots);
+bool vm_narrow_by_frames(int c_in, int c_out, int slots); /* the kernel takes VmLayerDev::frame_begin and frame_end */
 int vm_launch_conv_narrow(const VmBatchDev& B, const VmLayerDev& L, const float* in, float* out, hipStream_t stream,
                           const char** kernel_name);
 
