@@ -578,7 +578,12 @@ class Engine64:
         H = np.ascontiguousarray(Hoc, dtype=np.float64)
         r = m.lookup(H, lens)
         cap = int((r[:, 1] - r[:, 0]).sum()) if len(r) else 0
-        return m, H, cap, np.zeros((max(cap, 1), 2), np.float64), np.zeros((cap + 1, m.n_neighbours), np.int32), np.zeros(max(cap, 1), np.int32)
+        return m, H, cap, np.empty((max(cap, 1), 2), np.float64), np.empty((cap + 1, m.n_neighbours), np.int32), np.empty(max(cap, 1), np.int32)
+
+    @staticmethod
+    def _first(a, n):
+        """the first n rows, as an array of their own where they are much less than the whole"""
+        return a[:n] if 8 * n > 7 * len(a) else a[:n].copy()
 
     def project(self, mesh, Hoc, lens):
         m, H, cap, px, nb, gidx = self._buffers(mesh, Hoc, lens)
@@ -587,13 +592,13 @@ class Engine64:
 
     def classify(self, mesh, Hoc, lens, image, fcc):
         m, H, cap, px, nb, gidx = self._buffers(mesh, Hoc, lens)
-        cls = np.zeros((cap + 1, self.network.n_out), np.float64)
+        cls = np.empty((cap + 1, self.network.n_out), np.float64)
         img = np.ascontiguousarray(image)
         V = native.host_check(self._lib.vmh_engine_classify(self.ptr, m.ptr, _dp(H), C.byref(lens), img.ctypes.data, fcc, cap,
                                                             _dp(px), _ip(nb), _ip(gidx), _dp(cls)), self._lib)
         if V == 0:
             return dict(px=px[:0], nb=nb[:0], gidx=gidx[:0], cls=cls[:0])
-        return dict(px=px[:V].copy(), nb=nb[:V + 1].copy(), gidx=gidx[:V].copy(), cls=cls[:V + 1].copy())
+        return dict(px=self._first(px, V), nb=self._first(nb, V + 1), gidx=self._first(gidx, V), cls=self._first(cls, V + 1))
 
     def __call__(self, mesh, Hoc, lens, image=None, fcc=None):
         if image is None:
