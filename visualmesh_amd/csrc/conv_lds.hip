@@ -460,8 +460,9 @@ int launch_lds(const VmBatchDev& B, const VmLayerDev& L, const float* in, float*
     /* the kernel addresses its input rows with 32-bit byte offsets */
     if ((uint64_t) B.n_row_tiles * VMHIP_TILE * C_IN * 4 > 0xffffffffull) return -1;
     /* Two or more blocks of 8 waves per CU where LDS allows (registers are capped at 128 per lane, four waves
-     * per SIMD); otherwise one block of 16 waves. */
-    constexpr bool single = 2 * lds > 160 * 1024;
+     * per SIMD); otherwise one block of 16 waves. So also for pairs of bf16 made from sampled rows: eight waves, with two blocks of rows each, spill 16 of their
+     * 128 registers there (4 -> 64 on 1.85 million rows 192 us, 176 so; fp32 rows 177 / 178; two such blocks per CU, at 64 registers, spill 35: 321). */
+    constexpr bool single = 2 * lds > 160 * 1024 || (C_IN == 4 && OUT_FMT == VM_ROWS_BF16X2);
     constexpr int NW = single ? 16 : 8;
     auto kernel = vm_conv_lds_kernel<C_IN, C_OUT_T, SLOTS, NW, HALO, OUT_FMT>;
     static std::atomic<bool> configured{false}; /* engines on several host threads may get here together */
