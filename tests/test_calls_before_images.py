@@ -101,3 +101,27 @@ def test_calls_cut_short_or_left_open():
     engine._staged = [frame["mesh"]]
     engine.run()  # the call's frame is staged, its image there
     _same(engine.fetch_pinned()[0], want)
+
+
+def test_the_geometry_is_there_when_the_first_half_returns():
+    """Megabytes of geometry and nothing that would hold the host up behind the verdict (a small page-locked image, one layer): what the first half returns
+    is whole as it returns, in a block that still has another pose's geometry."""
+    rng, host = np.random.default_rng(5), native.host()
+    net = wl.glorot_network(np.random.default_rng(3), [3, 4], 6, wl.SELU)
+    engine, other = (eng.Engine(net, wl.RING6) for _ in range(2))
+    image = native.pinned_empty((256, 320), np.uint8)
+    image[:] = rng.integers(0, 256, image.shape, np.uint8)
+    mesh, lens = eng.Mesh(wl.RING6, wl.SPHERE, 0.0949, 1.0, 10.0, 20.0), native.make_lens(320, 256, wl.EQUISOLID, 105.0, math.pi)
+    wants = []
+    for pitch in (30.0, 50.0):
+        frame = dict(mesh=mesh, Hoc=wl.make_hoc(1.0, math.radians(pitch), 0.05, 0.3), lens=lens, image=image, fourcc=wl.fourcc("GREY"))
+        wants.append((frame, _staged(other, frame)))
+    for turn in range(6):
+        frame, want = wants[turn % 2]
+        V, r, H = len(want["gidx"]), native.Result(), np.ascontiguousarray(frame["Hoc"], np.float32)
+        assert V > 100000
+        native.host_check(host.vmh_engine_classify_begin(engine.ptr, mesh.ptr, H.ctypes.data_as(C.POINTER(C.c_float)), C.byref(lens), image.ctypes.data, frame["fourcc"], C.byref(r)))
+        nb, px, gidx = (np.ctypeslib.as_array(p, shape).copy() for p, shape in ((r.neighbourhood, (V + 1, 6)), (r.pixel_coordinates, (V, 2)), (r.global_indices, (V,))))
+        native.host_check(host.vmh_engine_classify_end(engine.ptr))
+        assert r.n_visible == V
+        _same(dict(px=px, nb=nb, gidx=gidx, cls=np.ctypeslib.as_array(r.classifications, (V + 1, 4))), want)

@@ -152,6 +152,7 @@ struct VmBatchDev {
     const VmDelivery* order; /* page-locked host memory; null beside a null delivery */
     VmDelivery* delivery;    /* the pass's copy of it; null: the batch's passes deliver nothing */
     uint32_t* published;     /* how many frames the pass's last kernel has published; it leaves zero */
+    uint32_t* stored;        /* how many of its blocks have stored their part of the results, where that is counted; it leaves zero */
     unsigned int* flow_timeouts; /* the batch's count of waits of the barrier-free kernel that ran out of polls (0 in a correct run) */
     /* edge guard: a candidate closer than amb_eps pixels to a screen edge is listed for the host's re-decision.
      * px_error is 0 outside tests: added to both pixel coordinates, it stands for a device whose lens arithmetic
@@ -267,6 +268,7 @@ struct VmPublish {
     int2* host_amb;
     uint32_t* host_timeouts;
     uint32_t* host_serial;    /* with the verdict: gets VmDelivery::serial when everything above is there */
+    uint32_t* host_stored;    /* gets VmDelivery::serial when the results are in the block too; null: nobody waits for that alone */
     const float* classes;     /* [rows][n_classes]; null while there are none */
     int32_t n_classes;        /* 0: the results have no classifications */
     uint8_t* classes_packed;  /* device memory with room for all classifications, to leave them there; null: into the block */
