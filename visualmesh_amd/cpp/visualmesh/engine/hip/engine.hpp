@@ -1071,8 +1071,9 @@ namespace engine {
                         if (s.busy) s.end();
                     } catch (...) {
                     }
-                    if (s.block) vmhip_host_free(s.block);
                 }
+                for (Home& h : homes_)
+                    if (h.block) vmhip_host_free(h.block);
             }
             Pipeline(const Pipeline&) = delete;
             Pipeline& operator=(const Pipeline&) = delete;
@@ -1084,20 +1085,22 @@ namespace engine {
                 Slot& now = slots_[step_ % 3];
                 Slot& oldest = slots_[(step_ + 1) % 3];
                 if (now.busy) now.end();  // an earlier call failed before it had waited for these
-                now.results.clear();
+                Home& home = homes_[step_ % homes_.size()];
+                home.results.clear();
+                now.home = &home;
                 now.submitted = true;
                 if (!frames.empty()) {
                     now.engine->stream_begin(frames, *slots_[0].engine);
                     now.busy = true, now.copied = false;
                     const size_t need = std::max<size_t>(now.engine->packed_size(), 256);
-                    if (need > now.block_bytes) {
-                        if (now.block) vmhip_host_free(now.block);
-                        now.block = vmhip_host_alloc(need + need / 8);
-                        now.block_bytes = now.block ? need + need / 8 : 0;
-                        if (!now.block) throw std::system_error(VMHIP_ERR_HIP, hip_error_category(), "Pipeline: no page-locked memory for the results");
+                    if (need > home.bytes) {
+                        if (home.block) vmhip_host_free(home.block);
+                        home.block = vmhip_host_alloc(need + need / 8);
+                        home.bytes = home.block ? need + need / 8 : 0;
+                        if (!home.block) throw std::system_error(VMHIP_ERR_HIP, hip_error_category(), "Pipeline: no page-locked memory for the results");
                     }
                     oldest.classes();  // ahead of the next copy in that direction
-                    now.engine->stream_geometry(now.block, now.block_bytes, now.results);
+                    now.engine->stream_geometry(home.block, home.bytes, home.results);
                     Slot& previous = slots_[(step_ + 2) % 3];
                     if (previous.busy) previous.engine->stream_images();  // one upload at a time
                     now.engine->stream_layers();
@@ -1127,12 +1130,16 @@ namespace engine {
             }
 
         private:
+            /// Where a batch's results go.
+            struct Home {
+                void* block = nullptr;
+                size_t bytes = 0;
+                std::vector<vmhip_result> results;
+            };
             struct Slot {
                 std::unique_ptr<Engine<Scalar>> engine;
+                Home* home = nullptr;
                 bool submitted = false, busy = false, copied = false;  ///< results to be returned; an engine at work for them; their last copy queued
-                void* block = nullptr;
-                size_t block_bytes = 0;
-                std::vector<vmhip_result> results;
                 void classes() {
                     if (busy && !copied) engine->stream_classes();
                     copied = true;
@@ -1151,13 +1158,16 @@ namespace engine {
                 const std::vector<vmhip_result>* done = nullptr;
                 const bool finish = oldest.submitted;
                 oldest.submitted = false;
-                if (finish) done = &oldest.results;
+                if (finish) done = &oldest.home->results;
                 if (previous.busy) previous.engine->stream_images();
                 if (oldest.busy) oldest.end();
                 return done;
             }
 
             std::array<Slot, 3> slots_;
+            /* One more than the engines: the geometry of a batch is on its way into its block in the call that begins the batch, and the results that
+             * the call before returned, of the batch three steps ago, are the caller's until that call is over. */
+            std::array<Home, 4> homes_;
             size_t step_ = 0;
         };
 
