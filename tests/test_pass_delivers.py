@@ -69,3 +69,24 @@ def test_the_last_two_layers_by_groups_of_frames(precision, frames, blind, halo_
             want = [{key: a.copy() for key, a in g.items()} for g in got]
         _same(got, want)
     _same(engine.fetch_pinned(), want)
+
+
+def test_no_groups_where_the_class_layer_could_not_be_launched_for_some_frames():
+    """Batches whose 64-wide rows reach 4 GiB, which the sliced class layer's 32-bit offsets do not: all frames at once. A first group that has fewer rows than the classifications of
+    the whole batch cover of the matrix beneath them would have the next one read rows that are no longer there."""
+    rng = np.random.default_rng(7)
+    small, lens, image = native.make_lens(320, 240, wl.EQUISOLID, 105.0, math.pi), native.make_lens(1280, 1280, wl.EQUIDISTANT, 400.0, math.pi), wl.random_image(rng, 1280, 1280, 4)
+    mesh, few = eng.Mesh(wl.RING6, wl.SPHERE, 0.0949, 1.0, 56.5, 20.0), eng.Mesh(wl.RING6, wl.SPHERE, 0.0949, 1.0, 2.0, 6.0)
+    batch = [dict(mesh=few, Hoc=wl.make_hoc(1.0, math.radians(30.0), 0.0, 0.0), lens=small, image=image[:240, :320].copy(), fourcc=wl.fourcc("RGBA"))]
+    batch += [dict(mesh=mesh, Hoc=wl.make_hoc(1.0, math.radians(90.0), 0.0, turn), lens=lens, image=image, fourcc=wl.fourcc("RGBA")) for turn in (0.3, 1.1)]
+    engine = eng.Engine(wl.glorot_network(np.random.default_rng(3), [3, 64, 64, 4], 6, wl.SELU), wl.RING6, native.BF16)
+    engine.stage(batch)
+    rows = [int((r[:, 1] - r[:, 0]).sum()) for r in (engine.staged_ranges(i) for i in range(3))]
+    assert sum(rows) * 64 * 4 > 1 << 32 and rows[0] * 8 < sum(rows) and rows[0] + rows[1] / 2 >= sum(rows) / 4
+    want = None
+    for turn in range(3):
+        engine.run()
+        got = engine.fetch_packed()
+        if want is None:
+            want = [{key: a.copy() for key, a in g.items()} for g in got]
+    _same(got, want)

@@ -361,7 +361,7 @@ hipError_t vm_flow_set_poll_limit(int polls); /* process wide; tests of the give
 /* layers with at most four output channels on v_mfma_f32_4x4x1 (64 rows x 4 channels per instruction), staged like
  * conv_flow.hip (conv_narrow.hip); reads the plain row-major weights */
 bool vm_narrow_supported(int c_in, int c_out, int slots);
-bool vm_narrow_by_frames(int c_in, int c_out, int slots); /* the kernel takes VmLayerDev::frame_begin and frame_end */
+bool vm_narrow_by_frames(const VmBatchDev& B, int c_in, int c_out, int slots); /* a kernel that takes VmLayerDev::frame_begin and frame_end can be launched for this batch */
 int vm_launch_conv_narrow(const VmBatchDev& B, const VmLayerDev& L, const float* in, float* out, hipStream_t stream,
                           const char** kernel_name);
 
