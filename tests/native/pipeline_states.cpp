@@ -202,9 +202,31 @@ int held() {
     return 0;
 }
 
+/* batches without frames, the first one among them */
+int empty() {
+    for (uint32_t first = 0; first < 4; ++first) {  // batches before the first empty one
+        Caller c;
+        uint32_t step = 0;
+        for (; step < first; ++step) CHECK(Caller::are(c.submit(10 + step, 2), 10 + step - 2, 2) == (step >= 2));
+        const Results* done = c.submit(0, 0);
+        CHECK(step >= 2 ? Caller::are(done, 10 + step - 2, 2) : done == nullptr);
+        CHECK(c.pipe.engine(int(step)).n_classes() == CLASSES);
+        for (++step; step < 8; ++step) {
+            done = c.submit(10 + step, 2);
+            if (step - 2 == first) CHECK(done && done->empty());
+            else if (step >= 2) CHECK(Caller::are(done, 10 + step - 2, 2));
+            else CHECK(done == nullptr);
+        }
+        CHECK(Caller::are(c.pipe.flush(), 16, 2));
+        CHECK(Caller::are(c.pipe.flush(), 17, 2));
+        CHECK(c.pipe.flush() == nullptr);
+    }
+    return 0;
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
-    const int rc = what == "held" ? held() : 2;
+    const int rc = what == "held" ? held() : what == "empty" ? empty() : 2;
     if (rc == 0) std::puts("ok");
     return rc;
 }

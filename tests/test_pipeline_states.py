@@ -22,3 +22,7 @@ def _run(program, what):
 
 def test_results_stay_until_two_more_calls(program):
     _run(program, "held")
+
+
+def test_batches_without_frames(program):
+    _run(program, "empty")

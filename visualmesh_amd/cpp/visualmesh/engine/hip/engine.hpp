@@ -348,6 +348,7 @@ namespace engine {
                 staging_ = false;
                 vmhip_engine* e = handle(N);
                 if (!batch_) throw_on_error(vmhip_batch_create(e, &batch_));
+                if (first && !first->batch_) throw_on_error(vmhip_batch_create(first->handle(N), &first->batch_));
                 const int32_t n = int32_t(flat.size());
                 if (n > 0)
                     throw_on_error(how == Stage::CALL     ? vmhip_batch_classify_begin(batch_, flat.data(), n, results->data())
@@ -422,7 +423,7 @@ namespace engine {
                 if (!results.empty()) throw_on_error(vmhip_batch_fetch_async(batch_, results.data()));
             }
             /// One batch of a stream of batches, by engines that take turns, step by step (see vmhip_batch_stream_begin; Pipeline takes them). `first` is the
-            /// same engine for all that take turns, has streamed a batch before the others do, and outlives them.
+            /// same engine for all that take turns, and outlives them.
             template <template <typename> class Model>
             std::vector<int32_t> stream_begin(const std::vector<Frame<Model>>& frames, const Engine& first) const {
                 std::vector<int32_t> visible(frames.size());
@@ -1104,6 +1105,9 @@ namespace engine {
                     Slot& previous = slots_[(step_ + 2) % 3];
                     if (previous.busy) previous.engine->stream_images();  // one upload at a time
                     now.engine->stream_layers();
+                }
+                else {
+                    now.engine->stage_async(frames);  // nothing to do, for an engine of this neighbour count
                 }
                 return advance();
             }
