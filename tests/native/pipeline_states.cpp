@@ -224,9 +224,57 @@ int empty() {
     return 0;
 }
 
+/* a step that fails: the batch is lost, the call that would have returned it says so (the call that submits it, if it never was under way), every other batch comes as it would have */
+int failures() {
+    const char* steps[] = {"begin", "layers", "images", "classes"};
+    for (const std::string step : steps)
+        for (uint32_t lost = 0; lost < 4; ++lost) {
+            const bool at_once = step == "begin" || step == "layers";
+            Caller c;
+            std::vector<uint32_t> order; /* what is under way, 0 for the batch that will be missing */
+            for (uint32_t turn = 0; turn < 9; ++turn) {
+                const uint32_t V = 10 + turn;
+                if (turn == lost && at_once) {
+                    failing = step;
+                    CHECK(c.throws(V, 2));
+                    continue; /* as if it had not been submitted */
+                }
+                order.push_back(turn == lost ? 0 : V);
+                if (order.size() > 2 && order[order.size() - 3] == 0) {
+                    failing = step == "classes" ? step : failing;
+                    CHECK(c.throws(V, 2));
+                    CHECK(failing.empty());
+                    continue;
+                }
+                const Results* done = c.submit(V, 2);
+                if (turn == lost && step == "images") failing = step; /* fails in the next call, is told by the one after that */
+                if (order.size() > 2) CHECK(Caller::are(done, order[order.size() - 3], 2));
+                else CHECK(done == nullptr);
+            }
+            CHECK(Caller::are(c.pipe.flush(), 17, 2));
+            CHECK(Caller::are(c.pipe.flush(), 18, 2));
+            CHECK(c.pipe.flush() == nullptr);
+            CHECK(c.pipe.flush() == nullptr);
+        }
+    /* while the pipeline drains, and behind that */
+    Caller c;
+    CHECK(c.submit(20, 2) == nullptr && c.submit(21, 3) == nullptr);
+    failing = "classes";
+    CHECK(c.flush_throws());
+    CHECK(Caller::are(c.pipe.flush(), 21, 3));
+    CHECK(c.pipe.flush() == nullptr);
+    failing = "begin";
+    CHECK(c.throws(22, 2));
+    CHECK(c.pipe.flush() == nullptr && c.pipe.flush() == nullptr && c.pipe.flush() == nullptr);
+    CHECK(c.submit(23, 2) == nullptr);
+    CHECK(Caller::are(c.pipe.flush(), 23, 2));
+    CHECK(c.pipe.flush() == nullptr);
+    return 0;
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
-    const int rc = what == "held" ? held() : what == "empty" ? empty() : 2;
+    const int rc = what == "held" ? held() : what == "empty" ? empty() : what == "failures" ? failures() : 2;
     if (rc == 0) std::puts("ok");
     return rc;
 }

@@ -26,3 +26,7 @@ def test_results_stay_until_two_more_calls(program):
 
 def test_batches_without_frames(program):
     _run(program, "empty")
+
+
+def test_a_step_that_fails(program):
+    _run(program, "failures")

@@ -1,5 +1,6 @@
 """Pipeline: geometry beside the upload, one copy at a time each way. What the ordinary test of it does not reach: overruled decisions, a batch cut short, an empty one."""
 import math
+import time
 
 import numpy as np
 import pytest
@@ -84,3 +85,36 @@ def test_overruled_decisions_and_a_batch_cut_short():
     del other  # with a batch under way
     fresh = eng.Pipeline(net, wl.RING6)
     _same(_through(fresh, batches), want)
+
+
+def test_batches_that_fail():
+    """One that cannot be queued is as if it had not been submitted, one whose network fails is lost and told in its turn; all others come as they would have."""
+    cfg, lib = wl.config(2, n_frames=1), native.hip()
+    batches = _batches(np.random.default_rng(5), [(4.0, 3.0), (6.0,), (4.0, 1.0), (3.0,), (2.0, 2.0)])
+    pipe, engine = eng.Pipeline(cfg.network, wl.RING6), eng.Engine(cfg.network, wl.RING6)
+    want = _wanted(engine, batches)
+
+    def submit(i):
+        done = pipe.submit(batches[i])
+        return None if done is None else [{k: v.copy() for k, v in r.items()} for r in done]
+
+    for _ in range(2):
+        assert submit(0) is None
+        native.hip_check(lib.vmhip_debug_set(native.DEBUG_CUT_SHORT, 1.0))
+        try:
+            with pytest.raises(native.VisualMeshError, match="cut short"):
+                submit(1)
+        finally:
+            native.hip_check(lib.vmhip_debug_set(native.DEBUG_CUT_SHORT, 0.0))
+        native.hip_check(lib.vmhip_debug_set(native.DEBUG_FLOW_POLL_LIMIT, 1))
+        try:
+            assert submit(1) is None
+            time.sleep(0.1)  # its network fails now
+        finally:
+            native.hip_check(lib.vmhip_debug_set(native.DEBUG_FLOW_POLL_LIMIT, 0))
+        _same([submit(2)], [want[0]])
+        with pytest.raises(native.VisualMeshError, match="gave up waiting"):
+            submit(3)
+        _same([submit(4)], [want[2]])
+        _same([pipe.flush(), pipe.flush()], want[3:])
+        assert pipe.flush() is None

@@ -506,6 +506,7 @@ void vmh_pipeline_destroy(vmh_pipeline* p) { delete p; }
 int vmh_pipeline_submit(vmh_pipeline* p, int n, const vmh_mesh* const* meshes, const real* Hoc16s, const vmh_lens_t* lenses,
                         const void* const* images, const uint32_t* fourccs) {
     GUARD({
+        p->done = nullptr;
         if (n == 0) p->done = p->pipe->flush();
         else if (p->model == VMH_RING6) {
             std::vector<HipEngine::Frame<Ring6>> frames(n);

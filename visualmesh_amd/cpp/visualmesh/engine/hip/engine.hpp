@@ -1067,12 +1067,7 @@ namespace engine {
                 for (Slot& s : slots_) s.engine.reset(new Engine<Scalar>(structure, precision));
             }
             ~Pipeline() {
-                for (Slot& s : slots_) {
-                    try {
-                        if (s.busy) s.end();
-                    } catch (...) {
-                    }
-                }
+                for (Slot& s : slots_) (void) s.end();
                 for (Home& h : homes_)
                     if (h.block) vmhip_host_free(h.block);
             }
@@ -1080,35 +1075,38 @@ namespace engine {
             Pipeline& operator=(const Pipeline&) = delete;
 
             /// Queue a batch; returns the results of the batch submitted two calls earlier (one entry per frame of that batch:
-            /// n_visible and pointers as in vmhip_result), or nullptr while the pipeline fills.
+            /// n_visible and pointers as in vmhip_result), or nullptr while the pipeline fills. A batch that cannot be queued is as if it had not been
+            /// submitted; one that fails later is lost, and the call that would have returned its results throws, with its own batch under way.
             template <template <typename> class Model>
             const std::vector<vmhip_result>* submit(const std::vector<typename Engine<Scalar>::template Frame<Model>>& frames) {
-                Slot& now = slots_[step_ % 3];
-                Slot& oldest = slots_[(step_ + 1) % 3];
-                if (now.busy) now.end();  // an earlier call failed before it had waited for these
+                Slot &now = slots_[step_ % 3], &oldest = slots_[(step_ + 1) % 3], &previous = slots_[(step_ + 2) % 3];
                 Home& home = homes_[step_ % homes_.size()];
-                home.results.clear();
-                now.home = &home;
-                now.submitted = true;
-                if (!frames.empty()) {
-                    now.engine->stream_begin(frames, *slots_[0].engine);
-                    now.busy = true, now.copied = false;
-                    const size_t need = std::max<size_t>(now.engine->packed_size(), 256);
-                    if (need > home.bytes) {
-                        if (home.block) vmhip_host_free(home.block);
-                        home.block = vmhip_host_alloc(need + need / 8);
-                        home.bytes = home.block ? need + need / 8 : 0;
-                        if (!home.block) throw std::system_error(VMHIP_ERR_HIP, hip_error_category(), "Pipeline: no page-locked memory for the results");
-                    }
-                    oldest.classes();  // ahead of the next copy in that direction
-                    now.engine->stream_geometry(home.block, home.bytes, home.results);
-                    Slot& previous = slots_[(step_ + 2) % 3];
-                    if (previous.busy) previous.engine->stream_images();  // one upload at a time
-                    now.engine->stream_layers();
+                if (frames.empty()) {
+                    now.engine->stage_async(frames);  // nothing to do, for an engine of this neighbour count
+                    home.results.clear();
                 }
                 else {
-                    now.engine->stage_async(frames);  // nothing to do, for an engine of this neighbour count
+                    now.engine->stream_begin(frames, *slots_[0].engine);
+                    now.busy = true, now.copied = false;
+                    try {
+                        const size_t need = std::max<size_t>(now.engine->packed_size(), 256);
+                        if (need > home.bytes) {
+                            if (home.block) vmhip_host_free(home.block);
+                            home.block = vmhip_host_alloc(need + need / 8);
+                            home.bytes = home.block ? need + need / 8 : 0;
+                            if (!home.block) throw std::system_error(VMHIP_ERR_HIP, hip_error_category(), "Pipeline: no page-locked memory for the results");
+                        }
+                        oldest.classes();  // ahead of the next copy in that direction
+                        now.engine->stream_geometry(home.block, home.bytes, home.results);
+                        previous.images();  // one upload at a time
+                        now.engine->stream_layers();
+                    } catch (...) {
+                        (void) now.end();
+                        throw;
+                    }
                 }
+                now.home = &home;
+                now.submitted = true;
                 return advance();
             }
             /// Drain: the results of the batches still in flight, oldest first, then nullptr.
@@ -1144,28 +1142,50 @@ namespace engine {
                 std::unique_ptr<Engine<Scalar>> engine;
                 Home* home = nullptr;
                 bool submitted = false, busy = false, copied = false;  ///< results to be returned; an engine at work for them; their last copy queued
+                std::exception_ptr failure;  ///< of a step of the batch at work, for the call that would return its results
+                template <typename Step>
+                void attempt(Step step) {
+                    if (!busy || failure) return;
+                    try {
+                        step();
+                    } catch (...) {
+                        failure = std::current_exception();
+                    }
+                }
+                void images() {
+                    attempt([this] { engine->stream_images(); });
+                }
                 void classes() {
-                    if (busy && !copied) engine->stream_classes();
+                    if (!copied) attempt([this] { engine->stream_classes(); });
                     copied = true;
                 }
-                void end() {
-                    const bool wait = busy;
-                    if (wait) classes();
+                /// leaves the engine with nothing under way; what has failed since the batch was begun
+                std::exception_ptr end() {
+                    classes();
+                    if (failure && busy) {
+                        try {
+                            engine->stream_classes();  // of a batch that is still under way: it is not, after that
+                        } catch (...) {
+                        }
+                    }
+                    std::exception_ptr before;
+                    std::swap(before, failure);
+                    attempt([this] { engine->stream_end(); });
+                    if (!before) std::swap(before, failure);
+                    failure = nullptr;
                     busy = false;
-                    if (wait) engine->stream_end();
+                    return before;
                 }
             };
             const std::vector<vmhip_result>* advance() {
                 Slot& previous = slots_[(step_ + 2) % 3];  // submitted one call ago: its images are to be read when this call returns
                 Slot& oldest = slots_[(step_ + 1) % 3];    // submitted two calls ago: to be finished
                 ++step_;
-                const std::vector<vmhip_result>* done = nullptr;
+                previous.images();
                 const bool finish = oldest.submitted;
                 oldest.submitted = false;
-                if (finish) done = &oldest.home->results;
-                if (previous.busy) previous.engine->stream_images();
-                if (oldest.busy) oldest.end();
-                return done;
+                if (const std::exception_ptr lost = oldest.end()) std::rethrow_exception(lost);
+                return finish ? &oldest.home->results : nullptr;
             }
 
             std::array<Slot, 3> slots_;

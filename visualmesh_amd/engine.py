@@ -385,7 +385,8 @@ class Pipeline:
     """visualmesh::engine::hip::Pipeline<float>: three engines in rotation behind one submit() call. submit(frames) queues a
     batch (images in page-locked memory, untouched until the next call returns) and returns the results of the batch
     submitted two calls earlier, or None while the pipeline fills; flush() drains (None when empty). The arrays returned
-    are views into the pipeline's page-locked memory, valid until two more calls."""
+    are views into the pipeline's page-locked memory, valid until two more calls. A batch that cannot be queued is as if it had not been
+    submitted; one that fails later is lost, and the call that would have returned it raises."""
 
     def __init__(self, network_groups, model, precision=native.FP32):
         self._lib = native.host()
@@ -394,8 +395,8 @@ class Pipeline:
         p = C.c_void_p()
         native.host_check(self._lib.vmh_pipeline_create(C.byref(self.network.c), model, precision, C.byref(p)))
         self.ptr = p
-        self._neighbours = []   # per batch in flight: the frames' neighbour counts
-        self._keep = []         # per batch in flight: what the asynchronous stage still reads
+        self._neighbours = 0    # of every node, as the last frames' meshes have it
+        self._keep = []         # of the last batches: what the asynchronous stage still reads
 
     def __del__(self):
         if getattr(self, "ptr", None):
@@ -405,8 +406,6 @@ class Pipeline:
     def _results(self, n_done, arrays=True):
         if n_done == 0:
             return None
-        nns = self._neighbours.pop(0)
-        self._keep.pop(0)
         if not arrays:
             return n_done
         n_out = self.network.n_out
@@ -414,7 +413,7 @@ class Pipeline:
         for i in range(n_done):
             px, gidx, nb, cls = C.POINTER(C.c_float)(), C.POINTER(C.c_int32)(), C.POINTER(C.c_int32)(), C.POINTER(C.c_float)()
             V = native.host_check(self._lib.vmh_pipeline_result(self.ptr, i, C.byref(px), C.byref(gidx), C.byref(nb), C.byref(cls)))
-            nn = nns[i]
+            nn = self._neighbours
             if V == 0:
                 out.append(dict(px=np.zeros((0, 2), np.float32), nb=np.zeros((0, nn), np.int32), gidx=np.zeros(0, np.int32), cls=np.zeros((0, n_out), np.float32)))
                 continue
@@ -433,8 +432,8 @@ class Pipeline:
         images = [np.ascontiguousarray(f["image"]) for f in frames]
         image_ptrs = (C.c_void_p * n)(*[im.ctypes.data for im in images])
         fccs = (C.c_uint32 * n)(*[f["fourcc"] for f in frames])
-        self._neighbours.append([m.n_neighbours for m in meshes])
-        self._keep.append(images)
+        self._neighbours = meshes[0].n_neighbours
+        self._keep = self._keep[-2:] + [images]
         return self._results(native.host_check(self._lib.vmh_pipeline_submit(self.ptr, n, mesh_ptrs, _fp(H), lenses, image_ptrs, fccs)), arrays)
 
     def graph_stats(self):
@@ -444,8 +443,6 @@ class Pipeline:
         return dict(captures=v[0].value, graph_launches=v[1].value, eager_launches=v[2].value)
 
     def flush(self, arrays=True):
-        if not self._neighbours:
-            return None
         return self._results(native.host_check(self._lib.vmh_pipeline_submit(self.ptr, 0, None, None, None, None, None)), arrays)
 
 
