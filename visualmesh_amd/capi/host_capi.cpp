@@ -292,13 +292,21 @@ int vmh_engine_time_calls(vmh_engine* e, const vmh_mesh* m, const real* Hoc16, c
 
 #if !defined(VMH_DOUBLE)
 /* The same two calls with the results left where the engine keeps them (vmhip_batch_fetch_held), for a caller that copies them
- * once into arrays of the right size, which it knows only now; a classification in two halves (vmhip_batch_classify_begin). Results of more than VMHIP_HELD_MOST bytes are not held: a projection
+ * once into arrays of the right size, which it knows only now; a classification also in two halves (vmhip_batch_classify_begin). Results of more than VMHIP_HELD_MOST bytes are not held: a projection
  * that may return so many is not run (n_visible -1, capacity the nodes of the lookup: vmh_engine_project does it), those of a
  * classification wait on the device with n_visible set and null pointers (vmhip_batch_fetch on the native batch brings them). */
 int vmh_engine_project_held(vmh_engine* e, const vmh_mesh* m, const real* Hoc16, const vmh_lens_t* lens, vmhip_result* result) {
     GUARD({
         *result = m->r6 ? e->engine->project_held(*m->r6, to_hoc(Hoc16), to_lens(lens), VMHIP_HELD_MOST)
                         : e->engine->project_held(*m->g8, to_hoc(Hoc16), to_lens(lens), VMHIP_HELD_MOST);
+        return 0;
+    })
+}
+int vmh_engine_classify_held(vmh_engine* e, const vmh_mesh* m, const real* Hoc16, const vmh_lens_t* lens, const void* image,
+                             uint32_t fourcc, vmhip_result* result) {
+    GUARD({
+        *result = m->r6 ? e->engine->classify_held(*m->r6, to_hoc(Hoc16), to_lens(lens), image, fourcc, VMHIP_HELD_MOST)
+                        : e->engine->classify_held(*m->g8, to_hoc(Hoc16), to_lens(lens), image, fourcc, VMHIP_HELD_MOST);
         return 0;
     })
 }

@@ -250,6 +250,23 @@ namespace engine {
             void classify_end() const {
                 if (batch_) throw_on_error(vmhip_batch_classify_end(batch_));
             }
+            /// Both halves in one: everything is there when it returns, in that block or, where the results are more than it may hold, in ordinary memory for
+            /// the one call (vmhip_batch_fetch_held). More than `most` bytes of results stay on the device: n_visible is set, the pointers are null.
+            template <template <typename> class Model>
+            vmhip_result classify_held(const Mesh<Scalar, Model>& mesh, const mat4<Scalar>& Hoc, const Lens<Scalar>& lens, const void* image, const uint32_t& format,
+                                       size_t most = std::numeric_limits<size_t>::max()) const {
+                vmhip_result r = classify_begin(mesh, Hoc, lens, image, format);
+                classify_end();
+                if (packed_size() > most) {
+                    const int32_t n_visible = r.n_visible;
+                    r = vmhip_result{};
+                    r.n_visible = n_visible;
+                }
+                else if (r.n_visible > 0 && !r.pixel_coordinates) {
+                    throw_on_error(vmhip_batch_fetch_held(batch_, &r));
+                }
+                return r;
+            }
             template <template <typename> class Model>
             ClassifiedMesh<Scalar, Model<Scalar>::N_NEIGHBOURS> operator()(const VisualMesh<Scalar, Model>& mesh,
                                                                            const mat4<Scalar>& Hoc,

@@ -330,6 +330,7 @@ def host():
     L.vmh_engine_destroy.argtypes = [vp]
     L.vmh_engine_destroy.restype = None
     L.vmh_engine_project_held.argtypes = [vp, vp, C.POINTER(C.c_float), C.POINTER(Lens), C.POINTER(Result)]
+    L.vmh_engine_classify_held.argtypes = [vp, vp, C.POINTER(C.c_float), C.POINTER(Lens), vp, C.c_uint32, C.POINTER(Result)]
     L.vmh_engine_classify_begin.argtypes = [vp, vp, C.POINTER(C.c_float), C.POINTER(Lens), vp, C.c_uint32, C.POINTER(Result)]
     L.vmh_engine_classify_end.argtypes = [vp]
     L.vmh_engine_project.argtypes = [vp, vp, C.POINTER(C.c_float), C.POINTER(Lens), C.c_int, C.POINTER(C.c_float),
