@@ -105,6 +105,16 @@ int main() {
     engine.fetch_wait();
     if (!same(got, want_large)) return std::puts("a run behind the streams"), 1;
     vmhip_host_free(block);
+
+    std::string names; /* of the kernels of a profiled pass: both parts of it */
+    if (vmhip_batch_profile(engine.native_batch(), 1) != VMHIP_OK || !stream(engine, large, want_large)) return std::puts("a profiled stream"), 1;
+    const char* name[16] = {};
+    float ms[16];
+    int64_t units[16];
+    int32_t n = 0;
+    if (vmhip_batch_profile_read(engine.native_batch(), 16, &n, name, ms, units) != VMHIP_OK) return std::puts("profile_read"), 1;
+    for (int i = 0; i < n; ++i) names += std::string(name[i]) + (ms[i] > 0.0f && ms[i] < 5.0f && units[i] > 0 ? " " : "? ");
+    if (names != "project compact neighbourhood sample ") return std::printf("profiled: %s\n", names.c_str()), 1;
     std::puts("ok");
     return 0;
 }
