@@ -1,4 +1,5 @@
-"""Pipeline: geometry beside the upload, one copy at a time each way. What the ordinary test of it does not reach: overruled decisions, a batch cut short, an empty one."""
+"""Pipeline: geometry beside the upload, one copy at a time each way. What the ordinary test of it does not reach: overruled decisions, batches that fail.
+(Empty batches, and results held across a call: test_pipeline_states.py.)"""
 import math
 import time
 
