@@ -271,8 +271,8 @@ int vmhip_batch_fetch_held(vmhip_batch* batch, vmhip_result* results);
  * device, as after vmhip_batch_run: n_visible is set, the pointers are NULL. No counterpart in the reference. */
 int vmhip_batch_classify_begin(vmhip_batch* batch, const vmhip_frame* frames, int32_t n_frames, vmhip_result* results);
 int vmhip_batch_classify_end(vmhip_batch* batch);
-/* One batch of a stream of batches, by engines that take turns: stream_begin stages the frames without their images and waits until the visible counts are known
- * (n_visible[n_frames]); stream_geometry queues the copy of everything but the classifications (block, bytes and results as for vmhip_batch_fetch_packed_async);
+/* One batch of a stream of batches, by engines that take turns: stream_begin waits for what is still under way on the batch's engine, stages the frames without their images
+ * and waits until the visible counts are known (n_visible[n_frames]); stream_geometry queues the copy of everything but the classifications (block, bytes and results as for vmhip_batch_fetch_packed_async);
  * stream_layers sends the images on their way (page-locked) and queues the network behind them; stream_images
  * waits until the images have been read; stream_classes waits for the network and queues the copy of the classifications; stream_end waits for all
  * copies. In this order, once each; until stream_end, or a failure of one of the others, the batch is used for nothing else. `first`: the same batch for all
